@@ -46,6 +46,7 @@
 
 #include <cstddef>
 #include <type_traits>
+#include <utility>
 
 namespace qh {
 
@@ -791,6 +792,21 @@ static int launch_gemm(GemmArgs a, qh_stream_t stream, const char* what) {
   return launch_status(what);
 }
 
+}  // namespace qh
+
+#include "gemm_small.h"
+
+namespace qh {
+
+// The tiling of the chunk's size (gemm_small::choose): every one computes
+// the same bits.
+template <int EPI, bool HW>
+static int dispatch_gemm(const GemmArgs& a, qh_stream_t stream, const char* what) {
+  const int v = gemm_small::choose(EPI, a.M, a.N, a.K);
+  return v < 0 ? launch_gemm<EPI, HW>(a, stream, what)
+               : gemm_small::launch_tiling<EPI, HW>(v, a, stream, what);
+}
+
 // Byte ranges the kernel addresses through 32-bit buffer offsets.
 static bool offsets_fit(int M, int N, int K, long lda, long ldb) {
   const long lim = 0x7fffffffL;
@@ -815,8 +831,8 @@ static int gemm_nt(const void* A, long lda, const float* sa, const void* B, long
   QH_REQUIRE(A && sa && B && sb && C, "%s: null pointer", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, C, ldc, nullptr,
              M, N, K, 0, 0, {}};
-  return hw ? launch_gemm<gemm::kStoreBf16, true>(a, stream, what)
-            : launch_gemm<gemm::kStoreBf16, false>(a, stream, what);
+  return hw ? dispatch_gemm<gemm::kStoreBf16, true>(a, stream, what)
+            : dispatch_gemm<gemm::kStoreBf16, false>(a, stream, what);
 }
 
 static int gemm_silu_quant(const void* A, long lda, const float* sa, const void* B, long ldb,
@@ -834,8 +850,8 @@ static int gemm_silu_quant(const void* A, long lda, const float* sa, const void*
   QH_REQUIRE(A && sa && B && sb && out_q && scales, "%s: null pointer", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, out_q, ld_out, scales,
              M, 2 * I, K, ue8m0, 0, {}};
-  return hw ? launch_gemm<gemm::kSiluQuant, true>(a, stream, what)
-            : launch_gemm<gemm::kSiluQuant, false>(a, stream, what);
+  return hw ? dispatch_gemm<gemm::kSiluQuant, true>(a, stream, what)
+            : dispatch_gemm<gemm::kSiluQuant, false>(a, stream, what);
 }
 
 static int gemm_qkv_rope(const void* A, long lda, const float* sa, const void* B, long ldb,
@@ -872,8 +888,8 @@ static int gemm_qkv_rope(const void* A, long lda, const float* sa, const void* B
                    (const uint16_t*)k_w, eps, n_q, n_kv, (uint16_t*)q_out, ld_q,
                    (uint16_t*)k_out, (uint16_t*)v_out, ld_kv, (uint16_t*)k_pool,
                    (uint16_t*)v_pool, row_dst, page_tokens};
-  return hw ? launch_gemm<gemm::kQkvRope, true>(a, stream, what)
-            : launch_gemm<gemm::kQkvRope, false>(a, stream, what);
+  return hw ? dispatch_gemm<gemm::kQkvRope, true>(a, stream, what)
+            : dispatch_gemm<gemm::kQkvRope, false>(a, stream, what);
 }
 
 extern "C" int qh_fp8_gemm_qkv_rope(const void* A, long lda, const float* sa, const void* B,

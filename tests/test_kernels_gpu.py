@@ -290,6 +290,69 @@ def test_fp8_gemm_silu_quant_ue8m0_matches_pair(M, I, Kd):
     assert torch.equal(q.view(torch.uint8).cpu(), q_pair.view(torch.uint8).cpu())
 
 
+# token counts at the edges of the GEMM's tilings (16, 32, 64 and 128 tokens)
+# and at sizes that take each of them
+TILING_SIZES = (1, 15, 16, 17, 33, 48, 64, 65, 100, 129, 200, 257, 400, 513, 700, 1025, 1300,
+                2049, 3000, 5000)
+
+
+def _head_rows(sa, m):
+    """The first m tokens' activation scales, column-major again."""
+    out = K.col_major_scales(m, sa.shape[1] * 128, sa.device)
+    out.copy_(sa[:m])
+    return out
+
+
+@pytest.mark.parametrize("ue8m0", [False, True])
+@pytest.mark.parametrize("epilogue,Kd", [("store", 128), ("store", 1152), ("store", 4224),
+                                         ("silu", 128), ("silu", 1152), ("qkv", 128),
+                                         ("qkv", 1152), ("qkv", 2560)])
+def test_fp8_gemm_bits_do_not_depend_on_the_chunk_size(epilogue, Kd, ue8m0):
+    """A token's output has one order of products and promotions whatever
+    tiling its chunk takes: the first m rows of an 18,000-token call (256 x
+    256 tiles) equal an m-token call bit for bit, for every epilogue, odd,
+    even and single K blocks, and both scale modes; arena pages included."""
+    n_q, n_kv, M = 32, 8, 18000
+    N = {"store": 2560, "silu": 5120, "qkv": (n_q + 2 * n_kv) * 128}[epilogue]
+    a, sa, w, sw = _gemm_inputs(21, M, N, Kd, DEV)
+    if ue8m0:
+        sa = sa.clone(memory_format=torch.preserve_format)
+        sa.copy_(torch.exp2(torch.ceil(torch.log2(sa))))
+        sw = torch.exp2(torch.ceil(torch.log2(sw)))
+    g = _gen(22)
+    pos = torch.randint(0, 5000, (M,), generator=g).to(DEV)
+    rope = (ref.rope_cache(4096, 128, 1e6).to(DEV),
+            (1 + 0.1 * torch.randn(128, generator=g)).to(torch.bfloat16).to(DEV),
+            (1 + 0.1 * torch.randn(128, generator=g)).to(torch.bfloat16).to(DEV), 1e-6, n_q, n_kv)
+    pages = M // 16 + 2
+    dst = (torch.arange(M) + 7).to(DEV)   # runs that start and end inside a page
+
+    def call(m):
+        args = (a[:m], _head_rows(sa, m), w, sw)
+        if epilogue == "store":
+            return [K.fp8_gemm_nt(*args, ue8m0_scales=ue8m0)]
+        if epilogue == "silu":
+            q, s = K.fp8_gemm_silu_quant(*args, ue8m0, ue8m0_scales=ue8m0)
+            return [q.view(torch.uint8), s.contiguous()]
+        rows = K.fp8_gemm_qkv_rope(*args, pos[:m].contiguous(), *rope, ue8m0_scales=ue8m0)
+        kp = torch.zeros(pages, n_kv, 16, 128, dtype=torch.bfloat16, device=DEV)
+        vp = torch.zeros(pages, n_kv, 128, 16, dtype=torch.bfloat16, device=DEV)
+        q = K.fp8_gemm_qkv_rope(*args, pos[:m].contiguous(), *rope, k_pool=kp, v_pool=vp,
+                                row_dst=dst[:m].contiguous(), ue8m0_scales=ue8m0)
+        assert torch.equal(q.view(torch.int16), rows[0].view(torch.int16))
+        k_rows, v_rows = layout.k_rows(kp), layout.v_rows(vp)
+        untouched = torch.cat([k_rows[:7], k_rows[m + 7:], v_rows[:7], v_rows[m + 7:]])
+        assert not untouched.view(torch.int16).any()
+        return list(rows) + [k_rows[7:m + 7], v_rows[7:m + 7]]
+
+    full = call(M)
+    for m in TILING_SIZES:
+        for i, (x, y) in enumerate(zip(call(m), full)):
+            bits = torch.uint8 if x.dtype == torch.uint8 else (
+                torch.int32 if x.dtype == torch.float32 else torch.int16)
+            assert torch.equal(x.contiguous().view(bits), y[:m].contiguous().view(bits)), (m, i)
+
+
 def test_fp8_gemm_silu_quant_oracle():
     """Against the oracle: fp64 GEMM rounded to bf16, then oracle silu_mul_quant."""
     g = _gen(13)
