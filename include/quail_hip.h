@@ -276,12 +276,9 @@ int qh_attention_fp8(const void* q, long ldq, int q_rows_total,
  * qh_attention_fp8 without the workspace argument, allocating nothing. No
  * counterpart in the reference: it is for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc). The q-tile scan goes to a static 512 KiB device array per GPU,
- * held until the process ends; its device address is looked up on the
- * first call on each device (the device current at the call must be the
- * stream's). At most 131072 sequences per call (QH_E_ARGUMENT beyond).
- * Calls that overlap on one GPU share that array and race; calls in order
- * on one stream do not. Output bit-identical to qh_attention_fp8.
+ * hipMalloc). The call holds no device memory of its own, so calls may
+ * overlap on one GPU. At most 131072 sequences per call (QH_E_ARGUMENT
+ * beyond). Output bit-identical to qh_attention_fp8.
  */
 int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_total,
                              const int64_t* q_rows, const void* k_pool,

@@ -16,7 +16,7 @@
 // V is transposed on its way into LDS).
 #include "common.h"
 
-#include <mutex>
+#include <algorithm>
 #include <type_traits>
 
 namespace qh {
@@ -65,7 +65,6 @@ struct AttnParams {
   long ldo;
   float* lse;
   long lse_stride;
-  const int32_t* tile_off;  // [n_seqs + 1] exclusive scan of q-tiles
   // fp8 output (attn_paged_kernel with FP8OUT): e4m3 [n_out, n_q*128] and
   // per-(row, head) scales [n_q, n_out]
   uint8_t* out_q;
@@ -74,41 +73,6 @@ struct AttnParams {
   int n_out;
   int ue8m0;
 };
-
-// Exclusive scan of per-sequence q-tile counts into tile_off[0..n_seqs].
-__global__ __launch_bounds__(1024) void attn_tile_scan_kernel(
-    const int32_t* __restrict__ cu_q, int n_seqs, int32_t* __restrict__ tile_off) {
-  __shared__ int32_t warp_sums[16];
-  __shared__ int32_t carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int base = 0; base < n_seqs; base += 1024) {
-    const int s = base + threadIdx.x;
-    int v = 0;
-    if (s < n_seqs) {
-      const int c = cu_q[s + 1] - cu_q[s];
-      v = c > 0 ? (c + attn::BQ - 1) / attn::BQ : 0;
-    }
-    // inclusive scan within the wave
-    int x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      int y = __shfl_up(x, o, 64);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) warp_sums[wid] = x;
-    __syncthreads();
-    int wave_off = 0;
-    for (int w = 0; w < wid; ++w) wave_off += warp_sums[w];
-    const int c0 = carry;
-    if (s < n_seqs) tile_off[s] = c0 + wave_off + x - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry = c0 + wave_off + x;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) tile_off[n_seqs] = carry;
-}
 
 // The node-resident tree kernel's two exclusive scans over the segments of
 // cu_a: q-tiles into tile_off[0..n_seg] and work into seg_cost[0..n_seg].
@@ -185,28 +149,45 @@ __global__ __launch_bounds__(1024) void attn_tree_scan_kernel(
   }
 }
 
-// The sequence of q-tile b: the largest s in [0, n) with off[s] <= b, where
-// off is non-decreasing and off[0] = 0 <= b. A 64-way search: each round the
-// wave's lanes load 64 evenly spaced candidates at once and a ballot picks
-// the last one <= b, so n <= 4096 takes two dependent loads where a binary
-// search of scalar loads takes twelve (each an L2 round trip, paid before a
-// workgroup can start its first DMA). Every lane of the wave must call it.
-template <typename T>
-__device__ __forceinline__ int last_le(const T* __restrict__ off, int n, T b, int lane) {
-  int lo = 0, span = n;  // off[lo] <= b; the answer lies in [lo, lo + span)
+// The largest s in [0, n) with key(s) <= b, where key is non-decreasing and
+// key(0) = 0 <= b. A 64-way search: each round the wave's lanes load 64 evenly
+// spaced candidates at once and a ballot picks the last one <= b, so n <= 4096
+// takes two dependent loads where a binary search of scalar loads takes twelve
+// (each an L2 round trip, paid before a workgroup can start its first DMA).
+// Every lane of the wave must call it.
+template <typename T, typename Key>
+__device__ __forceinline__ int last_le_key(int n, T b, int lane, Key key) {
+  int lo = 0, span = n;  // key(lo) <= b; the answer lies in [lo, lo + span)
   while (span > 1) {
     const int step = (span + 63) >> 6;
     const int idx = lo + lane * step;
-    const bool ok = lane * step < span && off[idx] <= b;
+    const bool ok = lane * step < span && key(idx) <= b;
     const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
-    const int k = 63 - __builtin_clzll(m);  // lane 0 always holds (off[lo] <= b)
+    const int k = 63 - __builtin_clzll(m);  // lane 0 always holds (key(lo) <= b)
     lo += k * step;
     span = min(step, span - k * step);
   }
   return __builtin_amdgcn_readfirstlane(lo);
 }
+template <typename T>
+__device__ __forceinline__ int last_le(const T* __restrict__ off, int n, T b, int lane) {
+  return last_le_key<T>(n, b, lane, [&](int i) { return off[i]; });
+}
 __device__ __forceinline__ int tile_seq(const int32_t* __restrict__ off, int n, int b, int lane) {
   return last_le<int32_t>(off, n, b, lane);
+}
+
+// The q-tiles of sequence s occupy slots seq_slot(s) .. of a launch of
+// n_queries / BQ + n_seqs slots: queries ahead of s, in whole tiles, plus one
+// slot per sequence ahead of it, which leaves room for s's own ceil(c / BQ)
+// tiles (floor((a + c) / BQ) - floor(a / BQ) + 1 >= ceil(c / BQ)). The slot is
+// read off cu directly, so no launch ahead of the attention counts tiles (a
+// 4-5 us kernel per layer); the slots between two sequences stay empty.
+__device__ __forceinline__ int seq_slot(const int32_t* __restrict__ cu, int s) {
+  return (int)((uint32_t)(cu[s] - cu[0]) / attn::BQ) + s;
+}
+__device__ __forceinline__ int slot_seq(const int32_t* __restrict__ cu, int n, int b, int lane) {
+  return last_le_key<int>(n, b, lane, [&](int i) { return seq_slot(cu, i); });
 }
 
 // The work item (q-tile b, head group y) of workgroup (bx, by). The hardware
@@ -264,13 +245,12 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnParams p) {
   // ---- which sequence and q-tile -------------------------------------------
   int b, hy;
   xcd_item(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, hy);
-  const int total_tiles = p.tile_off[p.n_seqs];
-  if (b >= total_tiles) return;
-  const int s = tile_seq(p.tile_off, p.n_seqs, b, lane);
+  const int s = slot_seq(p.cu_q, p.n_seqs, b, lane);
   const int q0 = p.cu_q[s];
   const int count = p.cu_q[s + 1] - q0;
   const int n_tiles = (count + BQ - 1) / BQ;
-  const int tq = n_tiles - 1 - (b - p.tile_off[s]);  // heaviest tile first
+  const int tq = n_tiles - 1 - (b - seq_slot(p.cu_q, s));  // heaviest tile first
+  if (tq < 0) return;
   const int i0 = tq * BQ;
   const int kv_len = p.kv_len[s];
 
@@ -563,13 +543,12 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
   // ---- sequence and q-tile (heaviest tile of a sequence first) -------------
   int b, hy;
   xcd_item(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, hy);
-  const int total_tiles = p.tile_off[p.n_seqs];
-  if (b >= total_tiles) return;
-  const int s = tile_seq(p.tile_off, p.n_seqs, b, lane);
+  const int s = slot_seq(p.cu_q, p.n_seqs, b, lane);
   const int q0 = p.cu_q[s];
   const int count = p.cu_q[s + 1] - q0;
   const int n_qt = (count + BQ - 1) / BQ;
-  const int i0 = (n_qt - 1 - (b - p.tile_off[s])) * BQ;
+  const int i0 = (n_qt - 1 - (b - seq_slot(p.cu_q, s))) * BQ;
+  if (i0 < 0) return;
   const int kv_len = p.kv_len[s];
   const int group = udiv_uniform(p.n_q, p.n_kv);
   const int hq = hy * HPW + wave;
@@ -904,8 +883,9 @@ struct TreeParams {
   long ld_out_q;
   float* out_scales;
   int ue8m0;
-  const int32_t* tile_off;    // [n_seg + 1] exclusive scan of q-tiles
-  const long long* seg_cost;  // [n_seg + 1] exclusive scan of work (node-resident kernel)
+  // the node-resident kernel's scans (attn_tree_scan_kernel)
+  const int32_t* tile_off;    // [n_seg + 1] q-tiles
+  const long long* seg_cost;  // [n_seg + 1] work
 };
 
 __device__ __forceinline__ int vswz(int key) { return 4 * (key & 3); }
@@ -926,13 +906,12 @@ __global__ __launch_bounds__(256, 3) void attn_tree_kernel(TreeParams p) {
   // ---- segment and q-tile (heaviest q-tile of a segment first) -------------
   int b, hy;
   xcd_item(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, hy);
-  const int total_tiles = p.tile_off[p.n_seg];
-  if (b >= total_tiles) return;
-  const int s = tile_seq(p.tile_off, p.n_seg, b, lane);
+  const int s = slot_seq(p.cu_a, p.n_seg, b, lane);
   const int q0 = p.cu_a[s];
   const int count = p.cu_a[s + 1] - q0;
   const int n_qt = (count + BQ - 1) / BQ;
-  const int i0 = (n_qt - 1 - (b - p.tile_off[s])) * BQ;
+  const int i0 = (n_qt - 1 - (b - seq_slot(p.cu_a, s))) * BQ;
+  if (i0 < 0) return;
   const int group = udiv_uniform(p.n_q, p.n_kv);
   const int hq = hy * HPW + wave;
   const int hk = udiv_uniform(hy * HPW, group);
@@ -1744,10 +1723,11 @@ __global__ __launch_bounds__(512, 1) void attn_tree_node_kernel(TreeParams p) {
 
 using namespace qh;
 
-// tile_off [n_seqs + 1] int32, then (node-resident tree calls) seg_cost
-// [n_seqs + 1] int64 at the next 16-byte boundary. The paged and streaming
-// calls use tile_off only (paged_workspace_bytes); the query returns what
-// every call needs.
+// The node-resident tree call's scans: tile_off [n_seqs + 1] int32, then
+// seg_cost [n_seqs + 1] int64 at the next 16-byte boundary. The other calls
+// read their q-tiles off cu_q and leave the workspace alone; they ask for
+// paged_workspace_bytes of it all the same, as callers were always told to
+// pass. The query returns what every call needs.
 static size_t seg_cost_offset(int n_seqs) {
   return ((size_t)(n_seqs + 1) * sizeof(int32_t) + 15) & ~(size_t)15;
 }
@@ -1805,12 +1785,7 @@ static int attention_launch(const void* q, long ldq, int q_rows_total, const int
   QH_REQUIRE(workspace && workspace_bytes >= paged_workspace_bytes(n_seqs),
              "attention: workspace of %zu bytes needed", paged_workspace_bytes(n_seqs));
   QH_REQUIRE(((uintptr_t)workspace & 15) == 0, "attention: workspace must be 16-byte aligned");
-  int32_t* tile_off = (int32_t*)workspace;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(attn_tile_scan_kernel, dim3(1), dim3(1024), 0, st, cu_q, n_seqs, tile_off);
-  int rc = launch_status("attention tile scan");
-  if (rc) return rc;
-
   AttnParams p;
   p.q = (const uint16_t*)q;
   p.ldq = ldq;
@@ -1835,15 +1810,13 @@ static int attention_launch(const void* q, long ldq, int q_rows_total, const int
   p.ldo = ldo;
   p.lse = lse;
   p.lse_stride = lse_stride;
-  p.tile_off = tile_off;
   p.out_q = (uint8_t*)out_q;
   p.ld_out_q = ld_out_q;
   p.out_scales = out_scales;
   p.n_out = n_queries;
   p.ue8m0 = ue8m0;
-  // upper bound on the q-tiles: sum ceil(c/32) <= n_queries/32 + n_seqs
-  const long max_tiles = (long)n_queries / attn::BQ + n_seqs;
-  dim3 grid((unsigned)max_tiles, (unsigned)(n_q / attn::HPW));
+  const long slots = (long)n_queries / attn::BQ + n_seqs;  // of q-tiles: seq_slot
+  dim3 grid((unsigned)slots, (unsigned)(n_q / attn::HPW));
   if (paged) {
     if (fp8) {
       if (causal) hipLaunchKernelGGL((attn_paged_kernel<true, true>), grid, dim3(256), 0, st, p);
@@ -1893,50 +1866,12 @@ extern "C" int qh_attention_fp8(const void* q, long ldq, int q_rows_total,
 }
 
 // ---------------------------------------------------------------------------
-// qh_attention_fp8_noalloc: qh_attention_fp8 with its q-tile scan in a
-// file-scope device array instead of a caller workspace, for callers that
-// cannot allocate. Each GPU holds its own copy of `scratch` (512 KiB) until
-// the process ends; its address on a device is looked up once, with that
-// device current, and kept per device. The scan kernel writes every entry
-// a launch reads (tile_off[0..n_seqs]), so nothing needs clearing between
-// calls. Calls that overlap on one GPU (two streams, two host threads)
-// share the array and race.
+// qh_attention_fp8_noalloc: qh_attention_fp8 without a workspace, for callers
+// that cannot allocate. The paged call needs none; the sequence limit is the
+// one this entry point has always had.
 namespace {
-
-constexpr int kScratchSeqs = 131072;               // sequences one call may carry
-constexpr int kScratchWords = kScratchSeqs + 128;  // + the scan's total and 256 B slack
-
-__device__ __align__(256) int32_t scratch[kScratchWords];
-
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mutex;
-int32_t* g_scratch_ptr[kMaxDevices] = {};
-
-// The current device's copy of `scratch` (its device address), looked up once.
-int scratch_on_current_device(int32_t** out) {
-  int dev = -1;
-  hipError_t err = hipGetDevice(&dev);
-  if (err != hipSuccess) {
-    set_error("attention_fp8_noalloc: hipGetDevice failed: %s", hipGetErrorString(err));
-    return QH_E_HIP;
-  }
-  QH_REQUIRE(dev >= 0 && dev < kMaxDevices, "attention_fp8_noalloc: device %d out of range",
-             dev);
-  std::lock_guard<std::mutex> lock(g_scratch_mutex);
-  if (g_scratch_ptr[dev] == nullptr) {
-    void* ptr = nullptr;
-    err = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (err != hipSuccess || ptr == nullptr) {
-      set_error("attention_fp8_noalloc: hipGetSymbolAddress(scratch) failed on device %d: %s",
-                dev, hipGetErrorString(err));
-      return QH_E_HIP;
-    }
-    g_scratch_ptr[dev] = static_cast<int32_t*>(ptr);
-  }
-  *out = g_scratch_ptr[dev];
-  return QH_OK;
-}
-
+constexpr int kNoAllocSeqs = 131072;  // sequences one call may carry
+alignas(16) char no_workspace[16];    // stands for a workspace; never dereferenced
 }  // namespace
 
 extern "C" int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_total,
@@ -1949,16 +1884,13 @@ extern "C" int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_tota
                                         float softmax_scale, int causal, void* out_q,
                                         long ld_out_q, float* scales, int ue8m0,
                                         qh_stream_t stream) {
-  QH_REQUIRE(n_seqs >= 0 && n_seqs <= kScratchSeqs,
+  QH_REQUIRE(n_seqs >= 0 && n_seqs <= kNoAllocSeqs,
              "attention_fp8_noalloc: %d sequences; the static scratch holds at most %d",
-             n_seqs, kScratchSeqs);
-  int32_t* ws = nullptr;
-  const int rc = scratch_on_current_device(&ws);
-  if (rc) return rc;
+             n_seqs, kNoAllocSeqs);
   return qh_attention_fp8(q, ldq, q_rows_total, q_rows, k_pool, v_pool, pool_pages, table,
                           table_width, page_tokens, cu_q, kv_len, n_seqs, n_queries, max_q,
                           n_q, n_kv, d, softmax_scale, causal, out_q, ld_out_q, scales, ue8m0,
-                          ws, (size_t)kScratchWords * sizeof(int32_t), stream);
+                          no_workspace, paged_workspace_bytes(n_seqs), stream);
 }
 
 // Shared by qh_tree_attention (streaming kernel) and
@@ -2006,21 +1938,22 @@ static int tree_attention_launch(const void* q, long ldq, int n_rows, const void
   QH_REQUIRE(workspace && workspace_bytes >= ws_need, "tree_attention: workspace of %zu bytes needed",
              ws_need);
   QH_REQUIRE(((uintptr_t)workspace & 15) == 0, "tree_attention: workspace must be 16-byte aligned");
-  int32_t* tile_off = (int32_t*)workspace;
-  long long* seg_cost = (long long*)((char*)workspace + seg_cost_offset(n_seg));
   hipStream_t st = (hipStream_t)stream;
   if (resident) {
     QH_REQUIRE((long)table_width * page_tokens <= ntree::RES * pattn::BKV,
                "tree_attention_resident: page-table rows of %d pages exceed the %d resident keys",
                table_width, ntree::RES * pattn::BKV);
   }
-  if (resident)
+  int32_t* tile_off = nullptr;
+  long long* seg_cost = nullptr;
+  if (resident) {
+    tile_off = (int32_t*)workspace;
+    seg_cost = (long long*)((char*)workspace + seg_cost_offset(n_seg));
     hipLaunchKernelGGL(attn_tree_scan_kernel, dim3(1), dim3(1024), 0, st, cu_a, seg_read,
                        read_used, n_reads, n_seg, tile_off, seg_cost);
-  else
-    hipLaunchKernelGGL(attn_tile_scan_kernel, dim3(1), dim3(1024), 0, st, cu_a, n_seg, tile_off);
-  int rc = launch_status("tree attention tile scan");
-  if (rc) return rc;
+    const int rc = launch_status("tree attention tile scan");
+    if (rc) return rc;
+  }
   TreeParams p;
   p.q = (const uint16_t*)q;
   p.ldq = ldq;
@@ -2057,9 +1990,8 @@ static int tree_attention_launch(const void* q, long ldq, int n_rows, const void
     else hipLaunchKernelGGL((attn_tree_node_kernel<false>), grid, dim3(512), 0, st, p);
     return launch_status("tree attention (node resident)");
   }
-  // upper bound on the q-tiles: sum ceil(c/32) <= n_rows/32 + n_seg
-  const long max_tiles = (long)n_rows / attn::BQ + n_seg;
-  dim3 grid((unsigned)max_tiles, (unsigned)(n_q / attn::HPW));
+  const long slots = (long)n_rows / attn::BQ + n_seg;  // of q-tiles: seq_slot
+  dim3 grid((unsigned)slots, (unsigned)(n_q / attn::HPW));
   if (fp8) hipLaunchKernelGGL((attn_tree_kernel<true>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((attn_tree_kernel<false>), grid, dim3(256), 0, st, p);
   return launch_status("tree attention");
