@@ -100,8 +100,10 @@ struct GemmArgs {
   const float* sb;
   void* C;        // bf16 [M, N] (kStoreBf16) or e4m3 [M, N/2] (kSiluQuant)
   long ldc;       // elements of C's type
-  float* scales;  // kSiluQuant: [N/256, M]
-  int M, N, K;
+  float* scales;  // kSiluQuant: [N/256, ld_sa]
+  int M, N, K;    // M: the end of the launch's tokens
+  int ld_sa;      // tokens per row of sa and scales: the whole call's
+  int row0;       // the launch's first token (gemm_small; 0 otherwise)
   int ue8m0;
   int group_m;    // tile rows per column sweep (see launch_gemm)
   QkvRope rope;   // kQkvRope only
@@ -216,7 +218,8 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_kernel(GemmArgs p) {
   const uint32_t offa = (uint32_t)(32 * wave + (lane >> 3)) * (uint32_t)lda +
                         (uint32_t)((((lane & 7) ^ (lane >> 3)) & 7) * 16);
   const uint32_t srow = 4u * (uint32_t)(32 * wave + (lane & 15));
-  const i32x4 rsa = buffer_rsrc(p.sa, (uint32_t)nk * (uint32_t)M * 4u);
+  const uint32_t ld_sa = (uint32_t)p.ld_sa;
+  const i32x4 rsa = buffer_rsrc(p.sa, (uint32_t)nk * ld_sa * 4u);
   const i32x4 rsb = buffer_rsrc(p.sb, (uint32_t)(p.N / 128) * (uint32_t)nk * 4u);
   struct ALoad {
     i32x4 ra;
@@ -227,7 +230,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_kernel(GemmArgs p) {
     const int m0 = c.tm * BM;
     L.ra = buffer_rsrc(p.A + (long)m0 * lda, (uint32_t)((long)min(M - m0, BM) * lda));
     L.k0 = (uint32_t)c.kb * BK;
-    L.ks = ((uint32_t)c.kb * (uint32_t)M + (uint32_t)m0) * 4u;
+    L.ks = ((uint32_t)c.kb * ld_sa + (uint32_t)m0) * 4u;
     L.kw0 = ((uint32_t)(weight_row(c.tn, 0) / 128) * (uint32_t)nk + (uint32_t)c.kb) * 4u;
     L.kw1 = ((uint32_t)(weight_row(c.tn, 1) / 128) * (uint32_t)nk + (uint32_t)c.kb) * 4u;
     return L;
@@ -577,7 +580,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_kernel(GemmArgs p) {
         acc[i][j] = zero;
         acc[i + 8][j] = zero;
       }
-      if (g == 0 && m_row + (lane & 15) < M) p.scales[(long)c.tn * M + m_row + (lane & 15)] = scale;
+      if (g == 0 && m_row + (lane & 15) < M) p.scales[(long)c.tn * p.ld_sa + m_row + (lane & 15)] = scale;
       // the 16 staged rows, eight whole 128-byte rows per instruction
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
@@ -798,13 +801,25 @@ static int launch_gemm(GemmArgs a, qh_stream_t stream, const char* what) {
 
 namespace qh {
 
-// The tiling of the chunk's size (gemm_small::choose): every one computes
+// The tilings of the chunk's size (gemm_small::choose): every one computes
 // the same bits.
 template <int EPI, bool HW>
 static int dispatch_gemm(const GemmArgs& a, qh_stream_t stream, const char* what) {
-  const int v = gemm_small::choose(EPI, a.M, a.N, a.K);
-  return v < 0 ? launch_gemm<EPI, HW>(a, stream, what)
-               : gemm_small::launch_tiling<EPI, HW>(v, a, stream, what);
+  const gemm_small::Plan plan = gemm_small::choose(EPI, a.M, a.N, a.K);
+  GemmArgs part = a;
+  part.ld_sa = a.M;
+  part.row0 = 0;
+  if (plan.large > 0) {
+    part.M = plan.large;
+    const int rc = launch_gemm<EPI, HW>(part, stream, what);
+    if (rc) return rc;
+  }
+  if (plan.large < a.M) {
+    part.M = a.M;
+    part.row0 = plan.large;
+    return gemm_small::launch_tiling<EPI, HW>(plan.small, part, stream, what);
+  }
+  return QH_OK;
 }
 
 // Byte ranges the kernel addresses through 32-bit buffer offsets.
@@ -830,7 +845,7 @@ static int gemm_nt(const void* A, long lda, const float* sa, const void* B, long
   if (M == 0) return QH_OK;
   QH_REQUIRE(A && sa && B && sb && C, "%s: null pointer", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, C, ldc, nullptr,
-             M, N, K, 0, 0, {}};
+             M, N, K, 0, 0, 0, 0, {}};
   return hw ? dispatch_gemm<gemm::kStoreBf16, true>(a, stream, what)
             : dispatch_gemm<gemm::kStoreBf16, false>(a, stream, what);
 }
@@ -849,7 +864,7 @@ static int gemm_silu_quant(const void* A, long lda, const float* sa, const void*
   if (M == 0) return QH_OK;
   QH_REQUIRE(A && sa && B && sb && out_q && scales, "%s: null pointer", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, out_q, ld_out, scales,
-             M, 2 * I, K, ue8m0, 0, {}};
+             M, 2 * I, K, 0, 0, ue8m0, 0, {}};
   return hw ? dispatch_gemm<gemm::kSiluQuant, true>(a, stream, what)
             : dispatch_gemm<gemm::kSiluQuant, false>(a, stream, what);
 }
@@ -883,7 +898,7 @@ static int gemm_qkv_rope(const void* A, long lda, const float* sa, const void* B
              "%s: null pointer", what);
   QH_REQUIRE(arena ? (k_pool && v_pool) : (k_out && v_out), "%s: null k/v destination", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, nullptr, 0, nullptr,
-             M, N, K, 0, 0, {}};
+             M, N, K, 0, 0, 0, 0, {}};
   a.rope = QkvRope{positions, (const uint16_t*)cos_sin, max_pos, (const uint16_t*)q_w,
                    (const uint16_t*)k_w, eps, n_q, n_kv, (uint16_t*)q_out, ld_q,
                    (uint16_t*)k_out, (uint16_t*)v_out, ld_kv, (uint16_t*)k_pool,

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
   // ---- tile: XCD-contiguous chunks, then group_m tile rows per column sweep --
   int tm, tn;
   {
-    const int tiles_m = (M + S::BM - 1) / S::BM;
+    const int tiles_m = (M - p.row0 + S::BM - 1) / S::BM;
     const int tiles_n = p.N / S::BR;
     const int per = (tiles_m * tiles_n) / gemm::XCDS;
     int t = (int)blockIdx.x;
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
     tm = first_m + (t % in_group) % gsize;
     tn = (t % in_group) / gsize;
   }
-  const int m0 = tm * S::BM;
+  const int m0 = p.row0 + tm * S::BM;
 
   // n-tile u of this wave, in the tile's row order. A fused epilogue wants a
   // column's partner in the same lane: gate n-tile i beside up n-tile i, a
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
   const i32x4 ra = buffer_rsrc(p.A + (long)m0 * p.lda,
                                (uint32_t)((long)min(M - m0, S::BM) * p.lda));
   const uint32_t offa = (uint32_t)(lane >> 3) * (uint32_t)p.lda + swz;
-  const i32x4 rsa = buffer_rsrc(p.sa, (uint32_t)nk * (uint32_t)M * 4u);
+  const i32x4 rsa = buffer_rsrc(p.sa, (uint32_t)nk * (uint32_t)p.ld_sa * 4u);
   const uint32_t offs = (uint32_t)lane * 4u;
   // DMA instruction op (0 .. LOADS - 1) of block kb into `stage`: weight
   // pieces, then activation pieces (every wave issues AL of them, the same
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
     } else {
       const int h = S::BM > 64 ? wave & 1 : 0;  // which 64 tokens
       const uint32_t dst = lds_addr(st + S::WBYTES + S::ABYTES + 256 * h);
-      const uint32_t so = ((uint32_t)kb * (uint32_t)M + (uint32_t)(m0 + 64 * h)) * 4u;
+      const uint32_t so = ((uint32_t)kb * (uint32_t)p.ld_sa + (uint32_t)(m0 + 64 * h)) * 4u;
       asm volatile(
           "s_mov_b32 m0, %0\n\t"
           "buffer_load_dword %1, %2, %3 offen lds"
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
                                      4 * g) =
             quant_e4m3_x4(acc[u][j][0], acc[u][j][1], acc[u][j][2], acc[u][j][3], rinv);
       const int m = m0 + tok0 + 16 * j + lane;
-      if (wr == 0 && g == 0 && m < M) p.scales[(long)tn * M + m] = scale;
+      if (wr == 0 && g == 0 && m < M) p.scales[(long)tn * p.ld_sa + m] = scale;
     }
     __syncthreads();
     uint8_t* out = (uint8_t*)p.C + (long)m0 * p.ldc + 128 * tn;
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
 template <int EPI, bool HW, int NR, int WT, int RT, int TM, int KU, int NS, int OCC>
 static int launch(GemmArgs a, qh_stream_t stream, const char* what) {
   using S = Shape<EPI, NR, WT, RT, TM, KU, NS>;
-  const int tiles = ((a.M + S::BM - 1) / S::BM) * (a.N / S::BR);
+  const int tiles = ((a.M - a.row0 + S::BM - 1) / S::BM) * (a.N / S::BR);
   a.group_m = 8;
   hipLaunchKernelGGL((fp8_gemm_small_kernel<EPI, HW, NR, WT, RT, TM, KU, NS, OCC>), dim3(tiles),
                      dim3(64 * S::NW), 0, (hipStream_t)stream, a);
@@ -521,62 +521,87 @@ static int launch(GemmArgs a, qh_stream_t stream, const char* what) {
 // block `first` us for the first round and `more` us for each further one
 // (shorter where two workgroups share a CU, longer where a full chip runs at a
 // lower clock). Fitted over the Qwen3-4B and Qwen3-32B projections at 1 to
-// 16,384 tokens (168 sizes, every tiling timed at each, one MI355X).
+// 40,000 tokens (248 sizes, every tiling timed at each, one MI355X).
 struct Tiling {
   int rows, tokens;
   float fixed, first, more;
 };
-constexpr Tiling kLarge[3] = {{256, 256, 2.4f, 1.28f, 1.80f},    // kStoreBf16
-                              {256, 256, 0.0f, 1.71f, 1.76f},    // kSiluQuant
-                              {256, 256, 10.5f, 1.24f, 1.94f}};  // kQkvRope
+constexpr Tiling kLarge[3] = {{256, 256, 2.7f, 1.288f, 1.784f},    // kStoreBf16
+                              {256, 256, 0.0f, 1.726f, 1.822f},    // kSiluQuant
+                              {256, 256, 11.9f, 1.214f, 1.975f}};  // kQkvRope
 constexpr int kTilings[3] = {7, 4, 5};
 constexpr Tiling kSmall[3][7] = {
-    {{32, 16, 4.0f, 0.111f, 0.132f},
-     {64, 16, 2.4f, 0.166f, 0.165f},
-     {64, 32, 2.5f, 0.194f, 0.198f},
-     {64, 64, 1.9f, 0.249f, 0.263f},
-     {128, 64, 0.4f, 0.415f, 0.290f},
-     {128, 128, 2.1f, 0.498f, 0.603f},
-     {256, 128, 1.4f, 0.780f, 0.994f}},
-    {{256, 16, 0.f, 0.709f, 0.575f},
-     {256, 32, 0.f, 0.801f, 0.699f},
-     {256, 64, 0.f, 0.903f, 0.772f},
-     {256, 128, 0.f, 1.162f, 1.102f}},
-    {{128, 16, 5.4f, 0.241f, 0.231f},
-     {128, 32, 6.6f, 0.262f, 0.237f},
-     {128, 64, 8.0f, 0.283f, 0.477f},
-     {128, 128, 11.4f, 0.413f, 0.761f},
-     {256, 128, 17.8f, 0.683f, 1.209f}}};
+    {{32, 16, 4.1f, 0.104f, 0.132f},
+     {64, 16, 2.6f, 0.161f, 0.162f},
+     {64, 32, 2.8f, 0.186f, 0.193f},
+     {64, 64, 2.4f, 0.245f, 0.268f},
+     {128, 64, 0.5f, 0.408f, 0.326f},
+     {128, 128, 3.1f, 0.498f, 0.629f},
+     {256, 128, 2.6f, 0.767f, 1.001f}},
+    {{256, 16, 0.f, 0.704f, 0.568f},
+     {256, 32, 0.f, 0.797f, 0.682f},
+     {256, 64, 0.f, 0.900f, 0.780f},
+     {256, 128, 0.f, 1.155f, 1.125f}},
+    {{128, 16, 5.8f, 0.222f, 0.238f},
+     {128, 32, 7.0f, 0.252f, 0.256f},
+     {128, 64, 8.6f, 0.267f, 0.484f},
+     {128, 128, 12.5f, 0.420f, 0.773f},
+     {256, 128, 20.2f, 0.624f, 1.208f}}};
 
-// The tiling with the lowest cost: an index into kSmall[EPI], or -1 for the
-// 256 x 256 kernel, which takes 8 % off its own cost, so that no size of the
-// fit runs slower than it does there (without it, four did, by up to 9 %).
-// Over those sizes the choice costs 0.1 % on average and 5 % at most against
-// the best measured tiling. Against 256 x 256 tiles alone (us, Qwen3-4B):
+// How a chunk's tokens are tiled: the first `large` on 256 x 256 tiles, the
+// rest, if any, on tiling `small` (an index into kSmall[epi]).
+struct Plan {
+  int large, small;
+};
+
+// The plan with the lowest cost, the small tilings' taken 10 % up (so that no
+// size of the fit runs slower than on 256 x 256 tiles alone; without it eight
+// did, by up to 9 %). With one tiling for all tokens the choice costs 0.02 %
+// on average and 2 % at most against the best measured one. Against 256 x 256
+// tiles alone (us, Qwen3-4B):
 //   tokens   qkv           o             gate_up       down
 //        1   32.8 ->  9.8  43.0 ->  6.9  31.9 -> 12.4  93.0 -> 11.3
 //       64   33.8 -> 10.5  42.9 ->  8.3  32.7 -> 14.9  94.4 -> 13.9
 //      256   36.3 -> 14.3  44.1 -> 10.7  33.1 -> 21.5  96.0 -> 19.4
-//     1024   37.0 -> 34.3  44.1 -> 20.4  68.1 -> 64.8  96.6 -> 39.6
+//     1024   37.0 -> 34.3  44.1 -> 20.4  68.1          96.6 -> 39.6
 //     2048   40.5          44.2 -> 28.5  103.6         95.8 -> 59.3
-//     8192   122.4         97.0 -> 89.2  354.2         229.1 -> 209.7
-static int choose(int epi, int M, int N, int K) {
+// Where the last round of 256 x 256 tiles would leave most of the chip idle,
+// its tokens go to a small tiling instead. Measured (us): o at 7,200 tokens, 290
+// tiles on 256 CUs, 100 -> 81 (6,400 tokens in one round, 800 on 128 x 128
+// tiles); down 224 -> 189, at 14,000 359 -> 328; Qwen3-32B at 3,200 tokens o 186
+// -> 138, down 577 -> 406; qkv at 2,600 tokens 75 -> 65.
+static Plan choose(int epi, int M, int N, int K) {
   const int nk = K / BK;
-  if (nk >= MAX_NK) return -1;  // the scale rows in LDS hold fewer blocks
+  if (nk >= MAX_NK) return {M, 0};  // the scale rows in LDS hold fewer blocks
   const int cus = device_cus();
-  auto cost = [&](const Tiling& t) {
-    const long tiles = (long)((M + t.tokens - 1) / t.tokens) * (N / t.rows);
+  auto cost = [&](const Tiling& t, int tokens) {
+    const long tiles = (long)((tokens + t.tokens - 1) / t.tokens) * (N / t.rows);
     const long rounds = (tiles + cus - 1) / cus;
     return t.fixed + (float)nk * (t.first + t.more * (float)(rounds - 1));
   };
-  int best = -1;
-  float least = 0.92f * cost(kLarge[epi]);
-  for (int i = 0; i < kTilings[epi]; ++i) {
-    const float c = cost(kSmall[epi][i]);
-    if (c < least) {
-      least = c;
-      best = i;
+  Plan best = {M, 0};
+  float least = cost(kLarge[epi], M);
+  auto with_small = [&](int large) {
+    const float ahead = large > 0 ? cost(kLarge[epi], large) : 0.f;
+    for (int i = 0; i < kTilings[epi]; ++i) {
+      const float c = ahead + 1.10f * cost(kSmall[epi][i], M - large);
+      if (c < least) {
+        least = c;
+        best = {large, i};
+      }
     }
+  };
+  with_small(0);
+  // whole rounds of 256 x 256 tiles, all but the last one or two
+  const Tiling& l = kLarge[epi];
+  const long columns = N / l.rows;
+  const long rounds = (long)(M / l.tokens) * columns / cus;
+  for (long r = rounds; r >= 1 && r >= rounds - 1; --r) {
+    // qkv past two rounds: the split measured -3 to +5 % (its long epilogues
+    // overlap the next tile's start in the persistent kernel)
+    if (epi == kQkvRope && r > 2) continue;
+    const long large = r * cus / columns * l.tokens;
+    if (large > 0 && large < M) with_small((int)large);
   }
   return best;
 }

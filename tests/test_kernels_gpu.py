@@ -290,10 +290,11 @@ def test_fp8_gemm_silu_quant_ue8m0_matches_pair(M, I, Kd):
     assert torch.equal(q.view(torch.uint8).cpu(), q_pair.view(torch.uint8).cpu())
 
 
-# token counts at the edges of the GEMM's tilings (16, 32, 64 and 128 tokens)
-# and at sizes that take each of them
+# token counts at the edges of the GEMM's tilings (16, 32, 64 and 128 tokens),
+# at sizes that take each of them, and at sizes split between 256 x 256 tiles
+# and a smaller tiling
 TILING_SIZES = (1, 15, 16, 17, 33, 48, 64, 65, 100, 129, 200, 257, 400, 513, 700, 1025, 1300,
-                2049, 3000, 5000)
+                2049, 3000, 3500, 5000, 7200, 14000)
 
 
 def _head_rows(sa, m):
