@@ -108,6 +108,20 @@ def load(path=LIB_PATH):
         return lib
 
 
+def load_ops():
+    """quail_amd._ops: the hot-path wrappers of kernels.py as native functions
+    (csrc/binding.cpp, linked to the kernel library)."""
+    import torch  # noqa: F401  (the module links to torch's libraries)
+
+    load()
+    try:
+        from quail_amd import _ops
+    except ImportError as err:
+        raise KernelLibraryMissing(
+            f"quail_amd/_ops.so is not built ({err}); run __graft_entry__.build()") from err
+    return _ops
+
+
 def exported_symbols():
     """The names the header declares, for the export check."""
     return tuple(SIGNATURES)

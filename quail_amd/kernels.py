@@ -2,14 +2,28 @@
 
 Each wrapper checks dtypes and layouts, allocates its outputs with torch on
 the input's device (kernels never allocate), and launches on the current
-torch stream. Activation scales come back the way the reference hands them
-to its GEMM: a (T, G) fp32 view of column-major (G, T) storage
+torch stream; the ones the layer loop calls do so in one native call
+(csrc/binding.cpp). Activation scales come back the way the reference hands
+them to its GEMM: a (T, G) fp32 view of column-major (G, T) storage
 (attention.py:153-156).
 """
 
 import torch
 
 from quail_amd import _hip
+
+
+class _Ops:
+    """The functions of quail_amd._ops, loaded at the first call, so that this
+    module imports where the libraries are not built."""
+
+    def __getattr__(self, name):
+        ops = _hip.load_ops()
+        self.__dict__.update({k: v for k, v in vars(ops).items() if not k.startswith("_")})
+        return getattr(ops, name)
+
+
+_ops = _Ops()
 
 GROUP = 128        # fp8 quant group, one MFMA K block (attention.py:30)
 PAGE_TOKENS = 16   # tokens per arena page (quail/cost/budgets.py:10)
@@ -46,20 +60,7 @@ def add_rmsnorm_quant(x, weight, eps, residual=None, ue8m0=False):
     The Triton add_rms_norm_quant (attention.py:325-359) with a residual,
     the layer-0 rms_norm + quant (attention.py:158-175) without one.
     """
-    _check(x, torch.bfloat16, "x", dim=2)
-    _check(weight, torch.bfloat16, "weight", dim=1)
-    T, H = x.shape
-    if residual is not None:
-        _check(residual, torch.bfloat16, "residual", dim=2)
-        if residual.shape != x.shape:
-            raise ValueError("residual shape differs from x")
-    q = torch.empty((T, H), dtype=torch.float8_e4m3fn, device=x.device)
-    scales = col_major_scales(T, H, x.device)
-    _hip.call("qh_add_rmsnorm_quant", _ptr(x), x.stride(0), _ptr(residual),
-              residual.stride(0) if residual is not None else 0, _ptr(weight),
-              float(eps), T, H, _ptr(q), _ptr(scales), int(bool(ue8m0)),
-              _stream())
-    return q, scales
+    return _ops.add_rmsnorm_quant(x, weight, eps, residual, ue8m0)
 
 
 def group_quant(x, ue8m0=False):
@@ -73,22 +74,6 @@ def group_quant(x, ue8m0=False):
     return q, scales
 
 
-def _check_gemm(a, a_scales, w, w_scales):
-    _check(a, torch.float8_e4m3fn, "a", dim=2)
-    _check(w, torch.float8_e4m3fn, "w", dim=2)
-    M, K = a.shape
-    N = w.shape[0]
-    if w.shape[1] != K:
-        raise ValueError(f"K mismatch: a {tuple(a.shape)} w {tuple(w.shape)}")
-    if a_scales.dtype != torch.float32 or tuple(a_scales.shape) != (M, K // GROUP) \
-            or (M > 1 and a_scales.stride(0) != 1) or (M > 0 and a_scales.stride(1) != M):
-        raise ValueError("a_scales must be a (M, K/128) view of column-major fp32")
-    if w_scales.dtype != torch.float32 or tuple(w_scales.shape) != (N // GROUP, K // GROUP) \
-            or not w_scales.is_contiguous():
-        raise ValueError("w_scales must be contiguous fp32 (N/128, K/128)")
-    return M, N, K
-
-
 def fp8_gemm_nt(a, a_scales, w, w_scales, out=None, ue8m0_scales=False):
     """out = (a * a_scales) (w * w_scales)^T in bf16 (DeepGEMM fp8_gemm_nt semantics).
 
@@ -97,13 +82,7 @@ def fp8_gemm_nt(a, a_scales, w, w_scales, out=None, ue8m0_scales=False):
     operands is a power of two, and the MFMA applies them itself
     (qh_fp8_gemm_nt_ue8m0).
     """
-    M, N, K = _check_gemm(a, a_scales, w, w_scales)
-    if out is None:
-        out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    _hip.call("qh_fp8_gemm_nt_ue8m0" if ue8m0_scales else "qh_fp8_gemm_nt", _ptr(a),
-              a.stride(0), _ptr(a_scales), _ptr(w), w.stride(0), _ptr(w_scales), _ptr(out),
-              out.stride(0), M, N, K, _stream())
-    return out
+    return _ops.fp8_gemm_nt(a, a_scales, w, w_scales, out, ue8m0_scales)
 
 
 def fp8_gemm_silu_quant(a, a_scales, w, w_scales, ue8m0=False, ue8m0_scales=False):
@@ -115,23 +94,7 @@ def fp8_gemm_silu_quant(a, a_scales, w, w_scales, ue8m0=False, ue8m0_scales=Fals
     ue8m0_scales: the input scales are powers of two, applied by the MFMA,
     and the output scales are UE8M0 too (qh_fp8_gemm_silu_quant_ue8m0).
     """
-    M, N, K = _check_gemm(a, a_scales, w, w_scales)
-    if N % (2 * GROUP):
-        raise ValueError(f"gate_up rows {N} must be a multiple of 256")
-    if ue8m0_scales and not ue8m0:
-        raise ValueError("ue8m0_scales=True writes UE8M0 output scales: pass ue8m0=True")
-    inter = N // 2
-    q = torch.empty((M, inter), dtype=torch.float8_e4m3fn, device=a.device)
-    scales = col_major_scales(M, inter, a.device)
-    if ue8m0_scales:
-        _hip.call("qh_fp8_gemm_silu_quant_ue8m0", _ptr(a), a.stride(0), _ptr(a_scales),
-                  _ptr(w), w.stride(0), _ptr(w_scales), M, inter, K, _ptr(q), q.stride(0),
-                  _ptr(scales), _stream())
-    else:
-        _hip.call("qh_fp8_gemm_silu_quant", _ptr(a), a.stride(0), _ptr(a_scales), _ptr(w),
-                  w.stride(0), _ptr(w_scales), M, inter, K, _ptr(q), q.stride(0),
-                  _ptr(scales), int(bool(ue8m0)), _stream())
-    return q, scales
+    return _ops.fp8_gemm_silu_quant(a, a_scales, w, w_scales, ue8m0, ue8m0_scales)
 
 
 def fp8_gemm_qkv_rope(a, a_scales, w, w_scales, positions, cos_sin, q_weight, k_weight, eps,
@@ -141,33 +104,8 @@ def fp8_gemm_qkv_rope(a, a_scales, w, w_scales, positions, cos_sin, q_weight, k_
     epilogue: fp8_gemm_nt then qk_norm_rope, bit for bit, without the qkv
     rows. Returns (q, k, v); with row_dst, k and v go to arena rows
     row_dst[m] of k_pool / v_pool instead and only q is returned."""
-    _check_gemm(a, a_scales, w, w_scales)
-    _check(cos_sin, torch.bfloat16, "cos_sin", dim=2)
-    M, K = a.shape
-    if w.shape[0] != (n_q + 2 * n_kv) * 128 or cos_sin.shape[1] != 128:
-        raise ValueError("qkv weight rows must be (n_q + 2 n_kv) * 128 with head_dim 128")
-    if positions.dtype != torch.int64 or positions.numel() != M or not positions.is_contiguous():
-        raise ValueError("positions must be contiguous int64, one per row")
-    dev = a.device
-    q = torch.empty((M, n_q * 128), dtype=torch.bfloat16, device=dev)
-    hw = int(bool(ue8m0_scales))
-    if row_dst is None:
-        k = torch.empty((M, n_kv * 128), dtype=torch.bfloat16, device=dev)
-        v = torch.empty((M, n_kv * 128), dtype=torch.bfloat16, device=dev)
-        _hip.call("qh_fp8_gemm_qkv_rope", _ptr(a), a.stride(0), _ptr(a_scales), _ptr(w),
-                  w.stride(0), _ptr(w_scales), M, K, n_q, n_kv, _ptr(positions),
-                  _ptr(cos_sin), cos_sin.shape[0], _ptr(q_weight), _ptr(k_weight),
-                  float(eps), _ptr(q), q.stride(0), _ptr(k), _ptr(v), k.stride(0), hw,
-                  _stream())
-        return q, k, v
-    if row_dst.dtype != torch.int64 or row_dst.numel() != M or not row_dst.is_contiguous():
-        raise ValueError("row_dst must be contiguous int64, one arena row per row")
-    _hip.call("qh_fp8_gemm_qkv_rope_kv", _ptr(a), a.stride(0), _ptr(a_scales), _ptr(w),
-              w.stride(0), _ptr(w_scales), M, K, n_q, n_kv, _ptr(positions), _ptr(cos_sin),
-              cos_sin.shape[0], _ptr(q_weight), _ptr(k_weight), float(eps), _ptr(q),
-              q.stride(0), _ptr(k_pool), _ptr(v_pool), _ptr(row_dst), PAGE_TOKENS, hw,
-              _stream())
-    return q
+    return _ops.fp8_gemm_qkv_rope(a, a_scales, w, w_scales, positions, cos_sin, q_weight, k_weight,
+                                  eps, n_q, n_kv, k_pool, v_pool, row_dst, ue8m0_scales)
 
 
 def qk_norm_rope(qkv, positions, cos_sin, q_weight, k_weight, eps, n_q, n_kv,
@@ -277,21 +215,8 @@ def attention_fp8(q3, cu_q, kv_len, *, n_queries, max_q, softmax_scale, causal,
     """Paged attention whose output is fp8-quantized per (row, head) in the
     kernel: (e4m3 [n_queries, n_q*d], scales (n_queries, n_q) column-major),
     bit-identical to group_quant(attention(...)) (attention.py:939-943, :798)."""
-    _check(q3, torch.bfloat16, "q", dim=3)
-    rows, n_q, d = q3.shape
-    if d != GROUP:
-        raise ValueError("one quant group per head needs head_dim 128")
-    n_seqs = cu_q.numel() - 1
-    dev = q3.device
-    q = torch.empty((n_queries, n_q * d), dtype=torch.float8_e4m3fn, device=dev)
-    scales = col_major_scales(n_queries, n_q * d, dev)
-    ws = torch.empty(_hip.workspace_bytes(n_seqs), dtype=torch.uint8, device=dev)
-    _hip.call("qh_attention_fp8", _ptr(q3), q3.stride(0), rows, _ptr(q_rows),
-              _ptr(k_pool), _ptr(v_pool), k_pool.shape[0], _ptr(table), table.shape[1],
-              PAGE_TOKENS, _ptr(cu_q), _ptr(kv_len), n_seqs, int(n_queries), int(max_q),
-              n_q, n_kv, d, float(softmax_scale), int(bool(causal)), _ptr(q), q.stride(0),
-              _ptr(scales), int(bool(ue8m0)), _ptr(ws), ws.numel(), _stream())
-    return q, scales
+    return _ops.attention_fp8(q3, cu_q, kv_len, n_queries, max_q, softmax_scale, causal, k_pool,
+                              v_pool, table, n_kv, q_rows, ue8m0)
 
 
 def tree_attention(q3, k_rows, v_rows, cu_a, seg_read, *, softmax_scale, k_pool=None,
@@ -309,40 +234,8 @@ def tree_attention(q3, k_rows, v_rows, cu_a, seg_read, *, softmax_scale, k_pool=
     Returns (e4m3 [T, n_q*d], scales (T, n_q) column-major) with fp8, else
     bf16 [T, n_q, d].
     """
-    _check(q3, torch.bfloat16, "q", dim=3)
-    _check(k_rows, torch.bfloat16, "k_rows", dim=3)
-    _check(v_rows, torch.bfloat16, "v_rows", dim=3)
-    T, n_q, d = q3.shape
-    n_kv = k_rows.shape[1]
-    if k_rows.shape[0] != T or v_rows.shape != k_rows.shape or k_rows.stride(0) != v_rows.stride(0):
-        raise ValueError("k_rows / v_rows must be [T, n_kv, d] with one row stride")
-    if k_rows.stride(1) != d or q3.stride(1) != d:
-        raise ValueError("heads of q / k_rows / v_rows must be contiguous")
-    n_seg = cu_a.numel() - 1
-    if seg_read.dtype != torch.int32 or seg_read.numel() != n_seg:
-        raise ValueError("seg_read must be int32 with one entry per segment")
-    dev = q3.device
-    n_reads = 0 if table is None else table.shape[0]
-    if n_reads and (used is None or used.numel() != n_reads):
-        raise ValueError("used must have one entry per page-table row")
-    ws = torch.empty(_hip.workspace_bytes(n_seg), dtype=torch.uint8, device=dev)
-    out = q = scales = None
-    if fp8:
-        if d != GROUP:
-            raise ValueError("one quant group per head needs head_dim 128")
-        q = torch.empty((T, n_q * d), dtype=torch.float8_e4m3fn, device=dev)
-        scales = col_major_scales(T, n_q * d, dev)
-    else:
-        out = torch.empty((T, n_q, d), dtype=torch.bfloat16, device=dev)
-    entry = "qh_tree_attention_resident" if resident else "qh_tree_attention"
-    _hip.call(entry, _ptr(q3), q3.stride(0), T, _ptr(k_rows), _ptr(v_rows),
-              k_rows.stride(0), _ptr(cu_a), _ptr(seg_read), n_seg,
-              _ptr(k_pool), _ptr(v_pool), 0 if k_pool is None else k_pool.shape[0],
-              _ptr(table), 0 if table is None else table.shape[1], _ptr(used), n_reads,
-              PAGE_TOKENS, n_q, n_kv, d, float(softmax_scale), _ptr(out),
-              0 if out is None else out.stride(0), _ptr(q), 0 if q is None else q.stride(0),
-              _ptr(scales), int(bool(ue8m0)), _ptr(ws), ws.numel(), _stream())
-    return (q, scales) if fp8 else out
+    return _ops.tree_attention(q3, k_rows, v_rows, cu_a, seg_read, softmax_scale, k_pool, v_pool,
+                               table, used, fp8, ue8m0, resident)
 
 
 def merge_attn_quant(out_a, lse_a, out_b, lse_b, source, ue8m0=False):
@@ -375,73 +268,30 @@ def silu_mul_quant(gate_up, ue8m0=False):
 
 def gather_rows(table, idx, out=None):
     """out[i] = table[idx[i]] for bf16 rows (embedding lookup, index_select)."""
-    _check(table, torch.bfloat16, "table", dim=2)
-    if idx.dtype != torch.int64 or not idx.is_contiguous():
-        raise ValueError("idx must be contiguous int64")
-    n, W = idx.numel(), table.shape[1]
-    if out is None:
-        out = torch.empty((n, W), dtype=torch.bfloat16, device=table.device)
-    _hip.call("qh_gather_rows", _ptr(table), table.stride(0), _ptr(idx), n, W,
-              _ptr(out), _stream())
-    return out
+    return _ops.gather_rows(table, idx, out)
 
 
 def gather_quant_rows(q, scales, idx):
     """Rows idx of an fp8 GEMM input and their 1x128 scales: (q[idx], scales[idx])
     with the scales in the same column-major (T, W/128) view."""
-    _check(q, torch.float8_e4m3fn, "q", dim=2)
-    T, W = q.shape
-    if scales.dtype != torch.float32 or scales.shape != (T, W // GROUP) or (
-            T > 0 and scales.stride() != (1, T)):
-        raise ValueError("scales must be the column-major (T, W/128) fp32 view")
-    if idx.dtype != torch.int64 or idx.dim() != 1 or not idx.is_contiguous():
-        raise ValueError("idx must be a contiguous 1-d int64 tensor")
-    n = idx.numel()
-    out = torch.empty((n, W), dtype=torch.float8_e4m3fn, device=q.device)
-    out_scales = col_major_scales(n, W, q.device)
-    _hip.call("qh_gather_quant_rows", _ptr(q), q.stride(0), _ptr(scales), T, _ptr(idx), n, W,
-              _ptr(out), out.stride(0), _ptr(out_scales), _stream())
-    return out, out_scales
+    return _ops.gather_quant_rows(q, scales, idx)
 
 
 def final_norm(hidden, residual, final_idx, weight, eps):
     """vLLM fused_add_rms_norm on the gathered answer rows (models/qwen3.py:119-124)."""
-    _check(hidden, torch.bfloat16, "hidden", dim=2)
-    _check(residual, torch.bfloat16, "residual", dim=2)
-    if not (hidden.is_contiguous() and residual.is_contiguous()):
-        raise ValueError("hidden and residual must be contiguous")
-    R, H = final_idx.numel(), hidden.shape[1]
-    out = torch.empty((R, H), dtype=torch.bfloat16, device=hidden.device)
-    _hip.call("qh_final_norm", _ptr(hidden), _ptr(residual), _ptr(final_idx), R,
-              H, _ptr(weight), float(eps), _ptr(out), _stream())
-    return out
+    return _ops.final_norm(hidden, residual, final_idx, weight, eps)
 
 
 def fused_add_rms_norm(hidden, residual, weight, eps):
     """vLLM fused_add_rms_norm in place (attention.py:177-181): residual <-
     hidden + residual, hidden <- RMSNorm(residual) * weight; returns both."""
-    _check(hidden, torch.bfloat16, "hidden", dim=2)
-    _check(residual, torch.bfloat16, "residual", dim=2)
-    if not (hidden.is_contiguous() and residual.is_contiguous()):
-        raise ValueError("hidden and residual must be contiguous")
-    if hidden.shape != residual.shape:
-        raise ValueError("hidden and residual shapes differ")
-    R, H = hidden.shape
-    _hip.call("qh_fused_add_rms_norm", _ptr(hidden), _ptr(residual), R, H, _ptr(weight),
-              float(eps), _stream())
+    _ops.fused_add_rms_norm(hidden, residual, weight, eps)
     return hidden, residual
 
 
 def answer_bits(normed, w_ans, is_true, with_margin=True):
     """TRUE/FALSE bit per row from the retained answer rows (readout.py:45-49, :70-79)."""
-    _check(normed, torch.bfloat16, "normed", dim=2)
-    R, H = normed.shape
-    bits = torch.empty(R, dtype=torch.uint8, device=normed.device)
-    margin = (torch.empty(R, dtype=torch.float32, device=normed.device)
-              if with_margin else None)
-    _hip.call("qh_answer_bits", _ptr(normed), R, H, _ptr(w_ans), w_ans.shape[0],
-              _ptr(is_true), _ptr(bits), _ptr(margin), _stream())
-    return bits, margin
+    return _ops.answer_bits(normed, w_ans, is_true, with_margin)
 
 
 def e4m3_encode(x):
@@ -455,10 +305,4 @@ def e4m3_encode(x):
 
 def answer_logits(normed, w_ans, is_true):
     """Per row, the best bf16 score of each class (readout.py:45-49)."""
-    _check(normed, torch.bfloat16, "normed", dim=2)
-    R, H = normed.shape
-    best_t = torch.empty(R, dtype=torch.bfloat16, device=normed.device)
-    best_f = torch.empty(R, dtype=torch.bfloat16, device=normed.device)
-    _hip.call("qh_answer_logits", _ptr(normed), R, H, _ptr(w_ans), w_ans.shape[0],
-              _ptr(is_true), _ptr(best_t), _ptr(best_f), _stream())
-    return best_t, best_f
+    return _ops.answer_logits(normed, w_ans, is_true)
