@@ -155,6 +155,19 @@ __device__ __forceinline__ uint32_t quant_e4m3_x4(float y0, float y1, float y2, 
   return (uint32_t)w;
 }
 
+// quant_e4m3_x4 with quant_e4m3's clamp to +-448, for values that a caller does
+// not know to be finite or within the group's maximum: the same bits as four
+// quant_e4m3 calls for every input, a NaN (clamped to -448) included.
+__device__ __forceinline__ uint32_t quant_e4m3_x4_clamped(float y0, float y1, float y2, float y3,
+                                                          double rinv) {
+  auto q = [&](float y) __attribute__((always_inline)) {
+    return fminf(fmaxf(div_exact(y, rinv), -kFp8Max), kFp8Max);
+  };
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(q(y0), q(y1), 0, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(q(y2), q(y3), w, true);
+  return (uint32_t)w;
+}
+
 // The maximum and the sum of a value and its partner lane's (lane ^ 32),
 // through v_permlane32_swap: the two halves of the wave trade values in one
 // VALU op instead of a ds_bpermute round trip through LDS. Both lanes of a
@@ -183,12 +196,6 @@ __device__ __forceinline__ float xor32_sum(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),
                                                   false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-__device__ __forceinline__ uint32_t quant_e4m3(float y, float scale) {
-  float q = div_exact(y, recip_exact(scale));
-  q = fminf(fmaxf(q, -kFp8Max), kFp8Max);
-  return f32_to_e4m3(q);
 }
 
 // silu(g) * u = g * sigmoid(g) * u in fp32 with sigmoid(g) = 1 / (1 + e^-g)
@@ -240,18 +247,37 @@ __device__ __forceinline__ float rope_second(float b, float a, float c, float s)
 
 // ---- lane reductions (wave64) -----------------------------------------------
 
-template <int WIDTH>
-__device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-  for (int o = 1; o < WIDTH; o <<= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
+// A value of another lane of the 16-lane row through a DPP move: a VALU operand
+// instead of a ds_bpermute round trip through LDS.
+template <int CTRL>
+__device__ __forceinline__ float row_lane(float v) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(
+      0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+// DPP controls of the butterfly's four steps within a row. Mirrors stand for
+// lane ^ 4 and lane ^ 8: the lanes of a quad (of a half row) hold the same bits
+// by then, so it does not matter which of them is read.
+constexpr int kXor1 = 0xb1;         // quad_perm [1, 0, 3, 2]
+constexpr int kXor2 = 0x4e;         // quad_perm [2, 3, 0, 1]
+constexpr int kHalfMirror = 0x141;  // lane i reads 7 - i of its half row
+constexpr int kMirror = 0x140;      // lane i reads 15 - i of its row
+
+// The maximum over the lane's 16-lane row.
+__device__ __forceinline__ float row_max(float v) {
+  v = fmaxf(v, row_lane<kXor1>(v));
+  v = fmaxf(v, row_lane<kXor2>(v));
+  v = fmaxf(v, row_lane<kHalfMirror>(v));
+  return fmaxf(v, row_lane<kMirror>(v));
 }
 
-template <int WIDTH>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int o = 1; o < WIDTH; o <<= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+// The sum over the wave: the butterfly over lane ^ 1, 2, 4, 8, 16, 32 (each
+// step adds two values, in either order the same bits).
+__device__ __forceinline__ float wave_sum(float v) {
+  v += row_lane<kXor1>(v);
+  v += row_lane<kXor2>(v);
+  v += row_lane<kHalfMirror>(v);
+  v += row_lane<kMirror>(v);
+  return xor32_sum(xor16_sum(v));
 }
 
 // 16-byte vector of 8 bf16.
@@ -259,6 +285,13 @@ struct alignas(16) bf16x8 {
   uint32_t w[4];
   __device__ __forceinline__ float get(int i) const {
     return bf16_to_f32((w[i >> 1] >> ((i & 1) * 16)) & 0xffffu);
+  }
+  // the pair (2 k, 2 k + 1) from fp32, each rounded to nearest even (NaN kept)
+  __device__ __forceinline__ void set_pair(int k, float a, float b) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    const f32x2_t x = {a, b};
+    w[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
   }
   __device__ __forceinline__ void set(int i, uint32_t bits) {
     uint32_t sh = (i & 1) * 16;

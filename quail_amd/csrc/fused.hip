@@ -19,6 +19,10 @@ namespace qh {
 // residual stores in flight. With the loads next to the residual stores and
 // these flags tested at run time, a wave made ten dependent HBM round trips
 // per row and waited for its own stores (0.31 ms for 102,400 rows of 2560).
+// Below a few thousand rows the wave's instruction chain is the bound: the
+// reductions run on DPP moves and the conversions take two values at a time
+// (834 vector instructions a row against 1,090: 41 rows 5.1 -> 4.4 us, 7,200
+// rows 21.2 -> 20.1 us).
 template <int VPL, bool FUSED, bool EXACT>
 __global__ __launch_bounds__(256) void add_rmsnorm_quant_kernel(
     const uint16_t* __restrict__ x, long ldx, uint16_t* __restrict__ residual,
@@ -67,12 +71,12 @@ __global__ __launch_bounds__(256) void add_rmsnorm_quant_kernel(
         const long col = ((long)i * 64 + lane) * 8;
         bf16x8 sum;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum.set(e, f32_to_bf16(v[i][e]));
+        for (int k = 0; k < 4; ++k) sum.set_pair(k, v[i][2 * k], v[i][2 * k + 1]);
         store8(residual + (long)t * ld_res + col, sum);
       }
     }
   }
-  ss = group_sum<64>(ss);
+  ss = wave_sum(ss);
   const float rstd = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
@@ -81,22 +85,22 @@ __global__ __launch_bounds__(256) void add_rmsnorm_quant_kernel(
       float y[8];
       float amax = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (FUSED) {
-          y[e] = v[i][e] * rstd * wv[i].get(e);
-        } else {
-          // vLLM rms_norm: bf16(bf16(x * rstd) * w)
-          y[e] = round_bf16(round_bf16(v[i][e] * rstd) * wv[i].get(e));
-        }
-        amax = fmaxf(amax, fabsf(y[e]));
+      for (int e = 0; e < 8; e += 2) {
+        float a = v[i][e] * rstd, b = v[i][e + 1] * rstd;
+        if (!FUSED) round_bf16_pair(a, b);  // vLLM rms_norm: bf16(bf16(x * rstd) * w)
+        a = a * wv[i].get(e);
+        b = b * wv[i].get(e + 1);
+        if (!FUSED) round_bf16_pair(a, b);
+        y[e] = a;
+        y[e + 1] = b;
+        amax = fmaxf(amax, fabsf(a));
+        amax = fmaxf(amax, fabsf(b));
       }
-      amax = group_max<16>(amax);
+      amax = row_max(amax);
       const float scale = group_scale(amax, ue8m0 != 0);
-      uint32_t lo = 0, hi = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) lo |= quant_e4m3(y[e], scale) << (8 * e);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) hi |= quant_e4m3(y[e + 4], scale) << (8 * e);
+      const double rinv = recip_exact(scale);
+      const uint32_t lo = quant_e4m3_x4_clamped(y[0], y[1], y[2], y[3], rinv);
+      const uint32_t hi = quant_e4m3_x4_clamped(y[4], y[5], y[6], y[7], rinv);
       uint2 packed = make_uint2(lo, hi);
       *reinterpret_cast<uint2*>(out_q + (long)t * H + col) = packed;
       if ((lane & 15) == 0) scales[(long)(col >> 7) * T + t] = scale;
@@ -120,13 +124,11 @@ __global__ __launch_bounds__(256) void group_quant_kernel(
   float amax = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(xv.get(e)));
-  amax = group_max<16>(amax);
+  amax = row_max(amax);
   const float scale = group_scale(amax, ue8m0 != 0);
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) lo |= quant_e4m3(xv.get(e), scale) << (8 * e);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) hi |= quant_e4m3(xv.get(e + 4), scale) << (8 * e);
+  const double rinv = recip_exact(scale);
+  const uint32_t lo = quant_e4m3_x4_clamped(xv.get(0), xv.get(1), xv.get(2), xv.get(3), rinv);
+  const uint32_t hi = quant_e4m3_x4_clamped(xv.get(4), xv.get(5), xv.get(6), xv.get(7), rinv);
   *reinterpret_cast<uint2*>(out_q + (long)t * W + col) = make_uint2(lo, hi);
   if (sub == 0) scales[(long)g * T + t] = scale;
 }
@@ -151,13 +153,11 @@ __global__ __launch_bounds__(256) void silu_mul_quant_kernel(
     y[e] = silu_mul(gv.get(e), uv.get(e));
     amax = fmaxf(amax, fabsf(y[e]));
   }
-  amax = group_max<16>(amax);
+  amax = row_max(amax);
   const float scale = group_scale(amax, ue8m0 != 0);
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) lo |= quant_e4m3(y[e], scale) << (8 * e);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) hi |= quant_e4m3(y[e + 4], scale) << (8 * e);
+  const double rinv = recip_exact(scale);
+  const uint32_t lo = quant_e4m3_x4_clamped(y[0], y[1], y[2], y[3], rinv);
+  const uint32_t hi = quant_e4m3_x4_clamped(y[4], y[5], y[6], y[7], rinv);
   *reinterpret_cast<uint2*>(out_q + (long)t * I + col) = make_uint2(lo, hi);
   if (sub == 0) scales[(long)g * T + t] = scale;
 }
@@ -428,13 +428,11 @@ __global__ __launch_bounds__(256) void merge_attn_quant_kernel(
   float amax = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(y[e]));
-  amax = group_max<16>(amax);
+  amax = row_max(amax);
   const float scale = group_scale(amax, ue8m0 != 0);
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) lo |= quant_e4m3(y[e], scale) << (8 * e);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) hi |= quant_e4m3(y[e + 4], scale) << (8 * e);
+  const double rinv = recip_exact(scale);
+  const uint32_t lo = quant_e4m3_x4_clamped(y[0], y[1], y[2], y[3], rinv);
+  const uint32_t hi = quant_e4m3_x4_clamped(y[4], y[5], y[6], y[7], rinv);
   *reinterpret_cast<uint2*>(out_q + (long)t * n_h * 128 + col) = make_uint2(lo, hi);
   if (sub == 0) scales[(long)h * T + t] = scale;
 }
@@ -476,6 +474,13 @@ __global__ __launch_bounds__(256) void gather_quant_rows_kernel(
 // lane reads its 8 columns of a row before it writes them, so out and
 // res_out may alias hidden and residual (the in-place vLLM form). One wave
 // per row.
+//
+// A chunk's answer rows are few (409 in a full one), so the kernel is bound by
+// the length of one wave's chain and not by bytes: VPL > 0 keeps the row's
+// sums in registers (H <= VPL * 512), so that every load is issued at once and
+// the second pass touches no memory (409 rows of 2560: 5.9 -> 4.4 us). VPL == 0 is the
+// two-pass form for any H.
+template <int VPL>
 __global__ __launch_bounds__(256) void final_norm_kernel(
     const uint16_t* hidden, const uint16_t* residual, const int64_t* __restrict__ idx,
     int R, int H, const uint16_t* __restrict__ w, float eps, uint16_t* out,
@@ -484,61 +489,126 @@ __global__ __launch_bounds__(256) void final_norm_kernel(
   if (i >= R) return;
   const int lane = threadIdx.x & 63;
   const long r = idx ? idx[i] : (long)i;
+  constexpr int V = VPL > 0 ? VPL : 1;
+  bf16x8 hv[V], rv[V], wv[V];
+  float z[V][8];
   float ss = 0.f;
-  for (int c = lane * 8; c < H; c += 512) {
-    bf16x8 hv = load8(hidden + r * H + c);
-    bf16x8 rv = load8(residual + r * H + c);
+  if constexpr (VPL > 0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float z = round_bf16(hv.get(e) + rv.get(e));
-      ss += z * z;
+    for (int k = 0; k < VPL; ++k) {
+      const int c = (k * 64 + lane) * 8;
+      if (c < H) {
+        hv[k] = load8(hidden + r * H + c);
+        rv[k] = load8(residual + r * H + c);
+        wv[k] = load8(w + c);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < VPL; ++k)
+      if ((k * 64 + lane) * 8 < H)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          z[k][e] = round_bf16(hv[k].get(e) + rv[k].get(e));
+          ss += z[k][e] * z[k][e];
+        }
+  } else {
+    for (int c = lane * 8; c < H; c += 512) {
+      hv[0] = load8(hidden + r * H + c);
+      rv[0] = load8(residual + r * H + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = round_bf16(hv[0].get(e) + rv[0].get(e));
+        ss += x * x;
+      }
     }
   }
-  ss = group_sum<64>(ss);
+  ss = wave_sum(ss);
   const float rstd = 1.0f / sqrtf(ss / (float)H + eps);
-  for (int c = lane * 8; c < H; c += 512) {
-    bf16x8 hv = load8(hidden + r * H + c);
-    bf16x8 rv = load8(residual + r * H + c);
-    bf16x8 wv = load8(w + c);
+  auto store = [&](int c, const float (&x)[8], const bf16x8& wc) __attribute__((always_inline)) {
     bf16x8 o, zr;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float z = round_bf16(hv.get(e) + rv.get(e));
-      zr.set(e, f32_to_bf16(z));
-      o.set(e, f32_to_bf16(round_bf16(z * rstd) * wv.get(e)));
+    for (int k = 0; k < 4; ++k) {
+      float a = x[2 * k] * rstd, b = x[2 * k + 1] * rstd;
+      round_bf16_pair(a, b);
+      zr.set_pair(k, x[2 * k], x[2 * k + 1]);
+      o.set_pair(k, a * wc.get(2 * k), b * wc.get(2 * k + 1));
     }
     if (res_out) store8(res_out + (long)i * H + c, zr);
     store8(out + (long)i * H + c, o);
+  };
+  if constexpr (VPL > 0) {
+#pragma unroll
+    for (int k = 0; k < VPL; ++k) {
+      const int c = (k * 64 + lane) * 8;
+      if (c < H) store(c, z[k], wv[k]);
+    }
+  } else {
+    for (int c = lane * 8; c < H; c += 512) {
+      hv[0] = load8(hidden + r * H + c);
+      rv[0] = load8(residual + r * H + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) z[0][e] = round_bf16(hv[0].get(e) + rv[0].get(e));
+      store(c, z[0], load8(w + c));
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
 // Answer readout: per row, bf16 scores against the retained answer rows,
-// strict TRUE > FALSE compare (readout.py:45-49, :70-79).
-__global__ __launch_bounds__(256) void answer_bits_kernel(
+// strict TRUE > FALSE compare (readout.py:45-49, :70-79). One workgroup per
+// row, wave w takes answers w, w + 4, .. two at a time: with one wave per row
+// the answers' dot products (each 2 H loads and a 64-lane sum) ran one after
+// the other, and 409 rows of 2560 against 8 answers took 12.2 us of which the
+// bytes need 1; now 4.6.
+constexpr int kAnswerWaves = 4;
+
+__global__ __launch_bounds__(64 * kAnswerWaves) void answer_bits_kernel(
     const uint16_t* __restrict__ normed, int R, int H,
     const uint16_t* __restrict__ w_ans, int n_ans,
     const uint8_t* __restrict__ is_true, uint8_t* __restrict__ bits,
     float* __restrict__ margin, uint16_t* __restrict__ best_true,
     uint16_t* __restrict__ best_false) {
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (i >= R) return;
+  __shared__ float best[kAnswerWaves][2];
+  const int i = blockIdx.x;
+  const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
+  const uint16_t* row = normed + (long)i * H;
   float best_t = -INFINITY, best_f = -INFINITY;
-  for (int a = 0; a < n_ans; ++a) {
-    float acc = 0.f;
-    for (int c = lane * 8; c < H; c += 512) {
-      bf16x8 nv = load8(normed + (long)i * H + c);
-      bf16x8 wv = load8(w_ans + (long)a * H + c);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc += nv.get(e) * wv.get(e);
-    }
-    acc = group_sum<64>(acc);
-    const float score = round_bf16(acc);
+  auto take = [&](int a, float acc) __attribute__((always_inline)) {
+    const float score = round_bf16(wave_sum(acc));
     if (is_true[a]) best_t = fmaxf(best_t, score);
     else best_f = fmaxf(best_f, score);
+  };
+  for (int a = wave; a < n_ans; a += 2 * kAnswerWaves) {
+    const int b = a + kAnswerWaves;
+    const uint16_t* wa = w_ans + (long)a * H;
+    const uint16_t* wb = w_ans + (long)(b < n_ans ? b : a) * H;
+    float acc_a = 0.f, acc_b = 0.f;
+#pragma unroll 5
+    for (int c = lane * 8; c < H; c += 512) {
+      const bf16x8 nv = load8(row + c);
+      const bf16x8 va = load8(wa + c);
+      const bf16x8 vb = load8(wb + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        acc_a += nv.get(e) * va.get(e);
+        acc_b += nv.get(e) * vb.get(e);
+      }
+    }
+    take(a, acc_a);
+    if (b < n_ans) take(b, acc_b);
   }
   if (lane == 0) {
+    best[wave][0] = best_t;
+    best[wave][1] = best_f;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 1; k < kAnswerWaves; ++k) {
+      best_t = fmaxf(best_t, best[k][0]);
+      best_f = fmaxf(best_f, best[k][1]);
+    }
     if (bits) bits[i] = best_t > best_f ? 1 : 0;
     if (margin) margin[i] = best_t - best_f;
     // the scores are bf16 values already: the top 16 bits are exact
@@ -746,17 +816,28 @@ extern "C" int qh_gather_quant_rows(const void* q, long ldq, const float* scales
   return launch_status("gather_quant_rows");
 }
 
+static int launch_final_norm(const void* hidden, const void* residual, const int64_t* idx, int R,
+                             int H, const void* w, float eps, void* out, void* res_out,
+                             qh_stream_t stream, const char* what) {
+  auto run = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(blocks_for(R, 4)), dim3(256), 0, (hipStream_t)stream,
+                       (const uint16_t*)hidden, (const uint16_t*)residual, idx, R, H,
+                       (const uint16_t*)w, eps, (uint16_t*)out, (uint16_t*)res_out);
+  };
+  if (H <= 5 * 512) run(final_norm_kernel<5>);
+  else if (H <= 10 * 512) run(final_norm_kernel<10>);
+  else run(final_norm_kernel<0>);
+  return launch_status(what);
+}
+
 extern "C" int qh_final_norm(const void* hidden, const void* residual,
                              const int64_t* final_idx, int R, int H, const void* w,
                              float eps, void* normed_out, qh_stream_t stream) {
   QH_REQUIRE(R >= 0 && H > 0 && H % 8 == 0, "final_norm: geometry");
   if (R == 0) return QH_OK;
   QH_REQUIRE(hidden && residual && final_idx && w && normed_out, "final_norm: null pointer");
-  hipLaunchKernelGGL(final_norm_kernel, dim3(blocks_for(R, 4)), dim3(256), 0,
-                     (hipStream_t)stream, (const uint16_t*)hidden,
-                     (const uint16_t*)residual, final_idx, R, H, (const uint16_t*)w, eps,
-                     (uint16_t*)normed_out, (uint16_t*)nullptr);
-  return launch_status("final_norm");
+  return launch_final_norm(hidden, residual, final_idx, R, H, w, eps, normed_out, nullptr, stream,
+                           "final_norm");
 }
 
 extern "C" int qh_fused_add_rms_norm(void* hidden, void* residual, int R, int H,
@@ -764,11 +845,8 @@ extern "C" int qh_fused_add_rms_norm(void* hidden, void* residual, int R, int H,
   QH_REQUIRE(R >= 0 && H > 0 && H % 8 == 0, "fused_add_rms_norm: geometry");
   if (R == 0) return QH_OK;
   QH_REQUIRE(hidden && residual && w, "fused_add_rms_norm: null pointer");
-  hipLaunchKernelGGL(final_norm_kernel, dim3(blocks_for(R, 4)), dim3(256), 0,
-                     (hipStream_t)stream, (const uint16_t*)hidden,
-                     (const uint16_t*)residual, (const int64_t*)nullptr, R, H,
-                     (const uint16_t*)w, eps, (uint16_t*)hidden, (uint16_t*)residual);
-  return launch_status("fused_add_rms_norm");
+  return launch_final_norm(hidden, residual, nullptr, R, H, w, eps, hidden, residual, stream,
+                           "fused_add_rms_norm");
 }
 
 extern "C" int qh_answer_bits(const void* normed, int R, int H, const void* w_ans,
@@ -777,7 +855,7 @@ extern "C" int qh_answer_bits(const void* normed, int R, int H, const void* w_an
   QH_REQUIRE(R >= 0 && H > 0 && H % 8 == 0 && n_ans > 0, "answer_bits: geometry");
   if (R == 0) return QH_OK;
   QH_REQUIRE(normed && w_ans && is_true && bits, "answer_bits: null pointer");
-  hipLaunchKernelGGL(answer_bits_kernel, dim3(blocks_for(R, 4)), dim3(256), 0,
+  hipLaunchKernelGGL(answer_bits_kernel, dim3(R), dim3(64 * kAnswerWaves), 0,
                      (hipStream_t)stream, (const uint16_t*)normed, R, H,
                      (const uint16_t*)w_ans, n_ans, is_true, bits, margin,
                      (uint16_t*)nullptr, (uint16_t*)nullptr);
@@ -801,7 +879,7 @@ extern "C" int qh_answer_logits(const void* normed, int R, int H, const void* w_
   if (R == 0) return QH_OK;
   QH_REQUIRE(normed && w_ans && is_true && best_true && best_false,
              "answer_logits: null pointer");
-  hipLaunchKernelGGL(answer_bits_kernel, dim3(blocks_for(R, 4)), dim3(256), 0,
+  hipLaunchKernelGGL(answer_bits_kernel, dim3(R), dim3(64 * kAnswerWaves), 0,
                      (hipStream_t)stream, (const uint16_t*)normed, R, H,
                      (const uint16_t*)w_ans, n_ans, is_true, (uint8_t*)nullptr,
                      (float*)nullptr, (uint16_t*)best_true, (uint16_t*)best_false);

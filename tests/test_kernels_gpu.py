@@ -713,6 +713,48 @@ def test_gather_final_norm_and_answer_bits():
         assert ((got.cpu().float() - want).abs() <= want.abs() * 2 ** -7 + 1e-3).all()
 
 
+@pytest.mark.parametrize("H", [8, 520, 2560, 2568, 5120, 5128, 8192])
+@pytest.mark.parametrize("R,n_ans", [(1, 1), (5, 2), (5, 9), (409, 8)])
+def test_final_norm_and_readout_at_every_width(R, n_ans, H):
+    """The register-held norm (H up to 2560 and 5120, partial last vectors) and
+    the two-pass one above it, gathered and in place, and the scores of 1 to 9
+    answers over the workgroup's waves, against the oracle."""
+    g = _gen(61 + R + H)
+    hidden = torch.randn(R + 3, H, generator=g).to(torch.bfloat16)
+    resid = torch.randn(R + 3, H, generator=g).to(torch.bfloat16)
+    w = (1 + 0.1 * torch.randn(H, generator=g)).to(torch.bfloat16)
+    fin = torch.randperm(R + 3, generator=g)[:R]
+    want, want_res = ref.fused_add_rms_norm(hidden, resid, w, 1e-6)
+    got = K.final_norm(hidden.to(DEV), resid.to(DEV), fin.to(DEV), w.to(DEV), 1e-6).cpu()
+    h_dev, r_dev = hidden.to(DEV), resid.to(DEV)
+    K.fused_add_rms_norm(h_dev, r_dev, w.to(DEV), 1e-6)
+    assert torch.equal(r_dev.cpu(), want_res)
+    # the same row takes the same bits through either entry point
+    assert torch.equal(h_dev.cpu()[fin], got)
+    # a sum in another order may move the inner rounding, bf16(z * rstd), by one
+    # bf16 step (at most 2^-7 of the value); times w, and with each side's outer
+    # rounding (2^-9 each, taken of the larger side), that is 2^-7 + 2^-8 at most
+    bound = torch.maximum(got.float().abs(), want[fin].float().abs()) * (2 ** -7 + 2 ** -8)
+    assert ((got.float() - want[fin].float()).abs() <= bound).all()
+    w_ans = (torch.randn(n_ans, H, generator=g) * 0.05).to(torch.bfloat16)
+    true = torch.arange(n_ans) % 2 == 0
+    best_t, best_f = K.answer_logits(got.to(DEV), w_ans.to(DEV), true.to(torch.uint8).to(DEV))
+    bits, margin = K.answer_bits(got.to(DEV), w_ans.to(DEV), true.to(torch.uint8).to(DEV))
+    scores = got.double() @ w_ans.double().t()
+    # fp32 sums of H products, each off by at most H * 2^-24 of the sum of
+    # magnitudes, then one bf16 rounding (2^-9)
+    bound = (got.double().abs() @ w_ans.double().abs().t()).amax(1) * H * 2 ** -24
+    for best, cols in ((best_t, true), (best_f, ~true)):
+        best = best.cpu().double()
+        if not cols.any():
+            assert torch.isinf(best).all() and (best < 0).all()
+            continue
+        top = scores[:, cols].amax(1)
+        assert ((best - top).abs() <= top.abs() * 2 ** -8 + bound).all()
+    assert torch.equal(bits.cpu().bool(), (best_t > best_f).cpu())
+    assert torch.equal(margin.cpu(), (best_t.float() - best_f.float()).cpu())
+
+
 # The two tree kernels: "stream" (qh_tree_attention, node pages streamed
 # per q-tile) and "node" (qh_tree_attention_resident, node K/V held in LDS;
 # page-table rows of at most 16 pages).
