@@ -15,6 +15,7 @@ import pytest
 import torch
 
 from oracle import ops as ref
+from quail_amd import _hip
 from quail_amd import kernels as K
 from quail_amd import layout
 
@@ -449,6 +450,45 @@ def test_paged_attention_ignores_unread_rows():
     assert torch.isfinite(got).all() and torch.isfinite(lse).all()
     assert (got - want).abs().max().item() <= 2e-3
     assert torch.allclose(lse, want_lse, atol=2e-3, rtol=0)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("n_seqs,prefix,max_suffix,n_q", [(1, 505, 3, 32), (1, 2049, 40, 32),
+                                                          (3, 1000, 33, 32), (8, 1600, 24, 64),
+                                                          (5, 4100, 70, 64)])
+def test_paged_attention_with_split_keys(n_seqs, prefix, max_suffix, n_q, causal):
+    """A few queries over long documents, whose keys are split over workgroups
+    and joined: against the oracle at the bar of the unsplit call, with a
+    document far shorter than the others (most of its splits are empty), NaN
+    in every arena row no sequence reads, and (not causal) a document of no
+    keys; the fp8 form equals the bf16 form quantized, bit for bit."""
+    case = _paged_case(300 + n_seqs + prefix, n_seqs, prefix, max_suffix, n_q=n_q)
+    T, width = int(case["cu_q"][-1]), case["table"].shape[1]
+    assert (_hip.paged_workspace_bytes(n_seqs, T, case["max_q"], width, n_q)
+            > _hip.workspace_bytes(n_seqs)), "the case does not split"
+    if n_seqs > 1:
+        case["used"][1] = case["lens"][1] + 17
+    if n_seqs > 2 and not causal:
+        case["used"][2] = 0
+    read = torch.zeros(case["k_rows"].shape[0], dtype=torch.bool)
+    for s in range(n_seqs):
+        j = torch.arange(int(case["used"][s]))
+        read[case["table"][s, j // 16].long() * 16 + j % 16] = True
+    case["k_rows"][~read] = float("nan")
+    case["v_rows"][~read] = float("nan")
+    got, lse, want, want_lse = _run_paged(case, causal=causal)
+    assert (got - want).abs().max().item() <= 2e-3
+    assert torch.allclose(lse, want_lse, atol=2e-3, rtol=0)
+    args = dict(n_queries=T, max_q=case["max_q"], softmax_scale=1 / math.sqrt(128), causal=causal,
+                k_pool=layout.k_pool_from_rows(case["k_rows"]).to(DEV),
+                v_pool=layout.v_pool_from_rows(case["v_rows"]).to(DEV),
+                table=case["table"].to(DEV), n_kv=case["n_kv"])
+    q_dev, cu, used = case["q"].to(DEV), case["cu_q"].to(DEV), case["used"].to(DEV)
+    out, _ = K.attention(q_dev, cu, used, **args)
+    for ue8m0 in (False, True):
+        q, sc = K.attention_fp8(q_dev, cu, used, ue8m0=ue8m0, **args)
+        rq, rs = K.group_quant(out.view(T, -1), ue8m0)
+        assert torch.equal(q.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(sc, rs)
 
 
 @pytest.mark.parametrize("causal,gathered", [(True, False), (False, True)])
