@@ -65,6 +65,7 @@ constexpr int STAGE = BR * BK;  // 32 KiB
 constexpr int A_WAVE = 32 * BK; // 4 KiB: a wave's 32 tokens of one K block
 constexpr int LOADS = 12;       // vector-memory loads per wave per step
 constexpr int XCDS = 8;
+constexpr int GROUP_M = 4;      // tile rows per column sweep (see launch_gemm)
 enum { kStoreBf16 = 0, kSiluQuant = 1, kQkvRope = 2 };
 }  // namespace gemm
 
@@ -101,9 +102,9 @@ struct GemmArgs {
   void* C;        // bf16 [M, N] (kStoreBf16) or e4m3 [M, N/2] (kSiluQuant)
   long ldc;       // elements of C's type
   float* scales;  // kSiluQuant: [N/256, ld_sa]
-  int M, N, K;    // M: the end of the launch's tokens
-  int ld_sa;      // tokens per row of sa and scales: the whole call's
-  int row0;       // the launch's first token (gemm_small; 0 otherwise)
+  int M, N, K;
+  int ld_sa;      // elements per row of sa and scales
+  int tile0, tiles;  // the launch's 256 x 256 tiles: tile0 .. tiles - 1 in tile order
   int ue8m0;
   int group_m;    // tile rows per column sweep (see launch_gemm)
   QkvRope rope;   // kQkvRope only
@@ -118,6 +119,16 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t bytes) {
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
+// Tile t of tiles_m x tiles_n in tile order: group_m tile rows per column sweep.
+__device__ __forceinline__ void tile_at(int t, int group_m, int tiles_m, int tiles_n, int& tm,
+                                        int& tn) {
+  const int in_group = group_m * tiles_n;
+  const int first_m = (t / in_group) * group_m;
+  const int gsize = min(tiles_m - first_m, group_m);
+  tm = first_m + (t % in_group) % gsize;
+  tn = (t % in_group) / gsize;
 }
 
 // silu(gate) * up of one GEMM output pair, with both rounded to bf16 first:
@@ -147,7 +158,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_kernel(GemmArgs p) {
   // ---- tiles of this workgroup --------------------------------------------
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = p.N / BR;
-  const int n_tiles = tiles_m * tiles_n;
+  const int n_tiles = p.tiles;  // from tile 0 on
   const int per_xcd = n_tiles / XCDS;
   const int G = gridDim.x;
   const int my_tiles = (n_tiles - (int)blockIdx.x + G - 1) / G;
@@ -157,11 +168,7 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_kernel(GemmArgs p) {
   const int group_m = p.group_m;
   auto coords = [&](int t, int& tm, int& tn) __attribute__((always_inline)) {
     if (t < per_xcd * XCDS) t = (t % XCDS) * per_xcd + t / XCDS;
-    const int in_group = group_m * tiles_n;
-    const int first_m = (t / in_group) * group_m;
-    const int gsize = min(tiles_m - first_m, group_m);
-    tm = first_m + (t % in_group) % gsize;
-    tn = (t % in_group) / gsize;
+    tile_at(t, group_m, tiles_m, tiles_n, tm, tn);
   };
   // first weight row of 128-row half h of tile column tn
   auto weight_row = [&](int tn, int h) __attribute__((always_inline)) {
@@ -786,10 +793,8 @@ __global__ __launch_bounds__(512, 1) void fp8_gemm_kernel(GemmArgs p) {
 // Qwen3-4B projection at 102,400 tokens, the fused gate_up included.
 template <int EPI, bool HW = false>
 static int launch_gemm(GemmArgs a, qh_stream_t stream, const char* what) {
-  const int tiles_n = a.N / gemm::BR;
-  const int tiles = ((a.M + gemm::BM - 1) / gemm::BM) * tiles_n;
-  const int grid = min(tiles, device_cus());
-  a.group_m = 4;
+  const int grid = min(a.tiles, device_cus());
+  a.group_m = gemm::GROUP_M;
   hipLaunchKernelGGL((fp8_gemm_kernel<EPI, HW>), dim3(grid), dim3(512), 0, (hipStream_t)stream,
                      a);
   return launch_status(what);
@@ -808,17 +813,16 @@ static int dispatch_gemm(const GemmArgs& a, qh_stream_t stream, const char* what
   const gemm_small::Plan plan = gemm_small::choose(EPI, a.M, a.N, a.K);
   GemmArgs part = a;
   part.ld_sa = a.M;
-  part.row0 = 0;
+  part.tile0 = 0;
+  part.tiles = plan.large;
   if (plan.large > 0) {
-    part.M = plan.large;
     const int rc = launch_gemm<EPI, HW>(part, stream, what);
     if (rc) return rc;
   }
-  if (plan.large < a.M) {
-    part.M = a.M;
-    part.row0 = plan.large;
+  part.tile0 = plan.large;
+  part.tiles = gemm_small::all_tiles(a.M, a.N);
+  if (part.tile0 < part.tiles)
     return gemm_small::launch_tiling<EPI, HW>(plan.small, part, stream, what);
-  }
   return QH_OK;
 }
 
@@ -845,7 +849,7 @@ static int gemm_nt(const void* A, long lda, const float* sa, const void* B, long
   if (M == 0) return QH_OK;
   QH_REQUIRE(A && sa && B && sb && C, "%s: null pointer", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, C, ldc, nullptr,
-             M, N, K, 0, 0, 0, 0, {}};
+             M, N, K, 0, 0, 0, 0, 0, {}};
   return hw ? dispatch_gemm<gemm::kStoreBf16, true>(a, stream, what)
             : dispatch_gemm<gemm::kStoreBf16, false>(a, stream, what);
 }
@@ -864,7 +868,7 @@ static int gemm_silu_quant(const void* A, long lda, const float* sa, const void*
   if (M == 0) return QH_OK;
   QH_REQUIRE(A && sa && B && sb && out_q && scales, "%s: null pointer", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, out_q, ld_out, scales,
-             M, 2 * I, K, 0, 0, ue8m0, 0, {}};
+             M, 2 * I, K, 0, 0, 0, ue8m0, 0, {}};
   return hw ? dispatch_gemm<gemm::kSiluQuant, true>(a, stream, what)
             : dispatch_gemm<gemm::kSiluQuant, false>(a, stream, what);
 }
@@ -898,7 +902,7 @@ static int gemm_qkv_rope(const void* A, long lda, const float* sa, const void* B
              "%s: null pointer", what);
   QH_REQUIRE(arena ? (k_pool && v_pool) : (k_out && v_out), "%s: null k/v destination", what);
   GemmArgs a{(const uint8_t*)A, lda, sa, (const uint8_t*)B, ldb, sb, nullptr, 0, nullptr,
-             M, N, K, 0, 0, 0, 0, {}};
+             M, N, K, 0, 0, 0, 0, 0, {}};
   a.rope = QkvRope{positions, (const uint16_t*)cos_sin, max_pos, (const uint16_t*)q_w,
                    (const uint16_t*)k_w, eps, n_q, n_kv, (uint16_t*)q_out, ld_q,
                    (uint16_t*)k_out, (uint16_t*)v_out, ld_kv, (uint16_t*)k_pool,

@@ -85,21 +85,25 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
   const int M = p.M;
   const int nk = p.K / BK;
 
-  // ---- tile: XCD-contiguous chunks, then group_m tile rows per column sweep --
+  // ---- tile: XCD-contiguous chunks, then group_m tile rows per column sweep;
+  // or the pieces, neighbours in launch order, of 256 x 256 tiles tile0 and up ----
   int tm, tn;
   {
-    const int tiles_m = (M - p.row0 + S::BM - 1) / S::BM;
-    const int tiles_n = p.N / S::BR;
-    const int per = (tiles_m * tiles_n) / gemm::XCDS;
+    constexpr int CM = gemm::BM / S::BM, CN = gemm::BR / S::BR;  // pieces of a 256 x 256 tile
+    const int n = (int)gridDim.x, per = n / gemm::XCDS;
     int t = (int)blockIdx.x;
     if (t < per * gemm::XCDS) t = (t % gemm::XCDS) * per + t / gemm::XCDS;
-    const int in_group = p.group_m * tiles_n;
-    const int first_m = (t / in_group) * p.group_m;
-    const int gsize = min(tiles_m - first_m, p.group_m);
-    tm = first_m + (t % in_group) % gsize;
-    tn = (t % in_group) / gsize;
+    if (p.tile0 == 0) {
+      tile_at(t, p.group_m, (M + S::BM - 1) / S::BM, p.N / S::BR, tm, tn);
+    } else {
+      tile_at(p.tile0 + t / (CM * CN), gemm::GROUP_M, (M + gemm::BM - 1) / gemm::BM,
+              p.N / gemm::BR, tm, tn);
+      tm = tm * CM + t % CM;
+      tn = tn * CN + t % (CM * CN) / CM;
+      if (tm * S::BM >= M) return;  // past the last token
+    }
   }
-  const int m0 = p.row0 + tm * S::BM;
+  const int m0 = tm * S::BM;
 
   // n-tile u of this wave, in the tile's row order. A fused epilogue wants a
   // column's partner in the same lane: gate n-tile i beside up n-tile i, a
@@ -510,7 +514,9 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
 template <int EPI, bool HW, int NR, int WT, int RT, int TM, int KU, int NS, int OCC>
 static int launch(GemmArgs a, qh_stream_t stream, const char* what) {
   using S = Shape<EPI, NR, WT, RT, TM, KU, NS>;
-  const int tiles = ((a.M - a.row0 + S::BM - 1) / S::BM) * (a.N / S::BR);
+  const int tiles = a.tile0 == 0
+                        ? ((a.M + S::BM - 1) / S::BM) * (a.N / S::BR)
+                        : (a.tiles - a.tile0) * (gemm::BM / S::BM) * (gemm::BR / S::BR);
   a.group_m = 8;
   hipLaunchKernelGGL((fp8_gemm_small_kernel<EPI, HW, NR, WT, RT, TM, KU, NS, OCC>), dim3(tiles),
                      dim3(64 * S::NW), 0, (hipStream_t)stream, a);
@@ -548,11 +554,22 @@ constexpr Tiling kSmall[3][7] = {
      {128, 128, 12.5f, 0.420f, 0.773f},
      {256, 128, 20.2f, 0.624f, 1.208f}}};
 
-// How a chunk's tokens are tiled: the first `large` on 256 x 256 tiles, the
-// rest, if any, on tiling `small` (an index into kSmall[epi]).
+// How a chunk is tiled: the first `large` 256 x 256 tiles, in tile order, as
+// such, the rest, if any, on tiling `small` (an index into kSmall[epi]).
 struct Plan {
   int large, small;
 };
+
+static int all_tiles(int M, int N) {
+  return ((M + gemm::BM - 1) / gemm::BM) * (N / gemm::BR);
+}
+
+// How many of the 256 x 256 tiles from tile `from` on are in the last tile row.
+static int last_row_tiles(int from, int M, int N) {
+  const int tiles_m = (M + gemm::BM - 1) / gemm::BM, tiles_n = N / gemm::BR;
+  const int first_m = (tiles_m - 1) / gemm::GROUP_M * gemm::GROUP_M;  // of the last group
+  return tiles_n - std::max(0, from - first_m * tiles_n) / (tiles_m - first_m);
+}
 
 // The plan with the lowest cost, the small tilings' taken 10 % up (so that no
 // size of the fit runs slower than on 256 x 256 tiles alone; without it eight
@@ -566,25 +583,35 @@ struct Plan {
 //     1024   37.0 -> 34.3  44.1 -> 20.4  68.1          96.6 -> 39.6
 //     2048   40.5          44.2 -> 28.5  103.6         95.8 -> 59.3
 // Where the last round of 256 x 256 tiles would leave most of the chip idle,
-// its tokens go to a small tiling instead. Measured (us): o at 7,200 tokens, 290
-// tiles on 256 CUs, 100 -> 81 (6,400 tokens in one round, 800 on 128 x 128
-// tiles); down 224 -> 189, at 14,000 359 -> 328; Qwen3-32B at 3,200 tokens o 186
-// -> 138, down 577 -> 406; qkv at 2,600 tokens 75 -> 65.
+// its tiles are cut into small ones in a second launch, which costs 8 us here
+// (its start, and a first round on cold LDS; with 4 two sizes ran up to 4 %
+// slower than unsplit). Tiles and not whole tile rows: gate_up has 76 tiles a
+// row. Measured (us, 256 x 256 tiles alone -> so): gate_up at 1,157 tokens, 380
+// tiles on 256 CUs, 69.3 -> 63.5, at 900 72 -> 58; o at 7,200 tokens, 290 tiles,
+// 99 -> 81; down 225 -> 185, at 14,000 358 -> 328; qkv at 3,000 75 -> 59;
+// Qwen3-32B at 4,000 tokens o 184 -> 154, down 578 -> 482.
 static Plan choose(int epi, int M, int N, int K) {
+  const int all = all_tiles(M, N);
   const int nk = K / BK;
-  if (nk >= MAX_NK) return {M, 0};  // the scale rows in LDS hold fewer blocks
+  if (nk >= MAX_NK) return {all, 0};  // the scale rows in LDS hold fewer blocks
   const int cus = device_cus();
-  auto cost = [&](const Tiling& t, int tokens) {
-    const long tiles = (long)((tokens + t.tokens - 1) / t.tokens) * (N / t.rows);
+  auto cost = [&](const Tiling& t, long tiles) {
     const long rounds = (tiles + cus - 1) / cus;
     return t.fixed + (float)nk * (t.first + t.more * (float)(rounds - 1));
   };
-  Plan best = {M, 0};
-  float least = cost(kLarge[epi], M);
+  // tiles of tiling t in the 256 x 256 tiles from `from` on
+  auto pieces = [&](const Tiling& t, int from) {
+    const int last = last_row_tiles(from, M, N);
+    const int tokens = M - (M - 1) / gemm::BM * gemm::BM;  // of the last tile row
+    return ((long)(all - from - last) * (gemm::BM / t.tokens) +
+            (long)last * ((tokens + t.tokens - 1) / t.tokens)) * (gemm::BR / t.rows);
+  };
+  Plan best = {all, 0};
+  float least = cost(kLarge[epi], all);
   auto with_small = [&](int large) {
-    const float ahead = large > 0 ? cost(kLarge[epi], large) : 0.f;
+    const float ahead = large > 0 ? cost(kLarge[epi], large) + 8.f : 0.f;
     for (int i = 0; i < kTilings[epi]; ++i) {
-      const float c = ahead + 1.10f * cost(kSmall[epi][i], M - large);
+      const float c = ahead + 1.10f * cost(kSmall[epi][i], pieces(kSmall[epi][i], large));
       if (c < least) {
         least = c;
         best = {large, i};
@@ -593,15 +620,12 @@ static Plan choose(int epi, int M, int N, int K) {
   };
   with_small(0);
   // whole rounds of 256 x 256 tiles, all but the last one or two
-  const Tiling& l = kLarge[epi];
-  const long columns = N / l.rows;
-  const long rounds = (long)(M / l.tokens) * columns / cus;
-  for (long r = rounds; r >= 1 && r >= rounds - 1; --r) {
+  const int rounds = all / cus;
+  for (int r = rounds; r >= 1 && r >= rounds - 1; --r) {
     // qkv past two rounds: the split measured -3 to +5 % (its long epilogues
     // overlap the next tile's start in the persistent kernel)
     if (epi == kQkvRope && r > 2) continue;
-    const long large = r * cus / columns * l.tokens;
-    if (large > 0 && large < M) with_small((int)large);
+    if (r * cus < all) with_small(r * cus);
   }
   return best;
 }

@@ -201,3 +201,20 @@ def test_no_unpadded_inline_asm_hazard(source, tmp_path):
     text = out.read_text()
     found = scan(text) + scan_tr_reads(text)
     assert not found, "\n".join(found[:10])
+
+
+@pytest.mark.skipif(not shutil.which(HIPCC) and not os.path.exists(HIPCC),
+                    reason="hipcc is not installed")
+@pytest.mark.parametrize("source", ["attention.hip", "gemm_fp8.hip"])
+def test_no_kernel_with_asm_loads_spills_vgprs(source, tmp_path):
+    """The compiler takes the outputs of a load in an asm statement as written
+    at once. Spilled, such a register is stored while its load is in flight and
+    then reused, and the load lands on the new value: an address, once, and the
+    access faulted. These sources keep asm loads in flight across steps, so
+    none of their kernels may use scratch memory."""
+    out = tmp_path / (source + ".s")
+    cmd = [HIPCC, *FLAGS, os.path.join(CSRC, source), "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True, cwd=CSRC, timeout=600)
+    text = out.read_text()
+    spills = re.findall(r"\.name:\s+(_Z\w+)(?:(?!\.name:).)*?\.vgpr_spill_count:\s+(\d+)", text, re.S)
+    assert spills and not [s for s in spills if s[1] != "0"], spills
