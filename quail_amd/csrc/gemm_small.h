@@ -579,11 +579,11 @@ constexpr Tiling kSmall[3][7] = {
      {256, 32, 0.f, 0.797f, 0.682f},
      {256, 64, 0.f, 0.900f, 0.780f},
      {256, 128, 0.f, 1.155f, 1.125f}},
-    {{128, 16, 5.8f, 0.222f, 0.238f},
-     {128, 32, 7.0f, 0.252f, 0.256f},
-     {128, 64, 8.6f, 0.267f, 0.484f},
-     {128, 128, 12.5f, 0.420f, 0.773f},
-     {256, 128, 20.2f, 0.624f, 1.208f}}};
+    {{128, 16, 4.3f, 0.236f, 0.249f},
+     {128, 32, 4.1f, 0.278f, 0.256f},
+     {128, 64, 5.5f, 0.314f, 0.469f},
+     {128, 128, 7.5f, 0.430f, 0.771f},
+     {256, 128, 10.2f, 0.672f, 1.249f}}};
 
 // How a chunk is tiled: the first `large` 256 x 256 tiles, in tile order, as
 // such, the rest, if any, on tiling `small` (an index into kSmall[epi]).
@@ -608,10 +608,10 @@ static int last_row_tiles(int from, int M, int N) {
 // on average and 2 % at most against the best measured one. Against 256 x 256
 // tiles alone (us, Qwen3-4B):
 //   tokens   qkv           o             gate_up       down
-//        1   32.8 ->  9.8  43.0 ->  6.9  31.9 -> 12.4  93.0 -> 11.3
-//       64   33.8 -> 10.5  42.9 ->  8.3  32.7 -> 14.9  94.4 -> 13.9
-//      256   36.3 -> 14.3  44.1 -> 10.7  33.1 -> 21.5  96.0 -> 19.4
-//     1024   37.0 -> 34.3  44.1 -> 20.4  68.1          96.6 -> 39.6
+//        1   33.4 ->  8.8  43.0 ->  6.9  31.9 -> 12.4  93.0 -> 11.3
+//       64   34.0 ->  9.3  42.9 ->  8.3  32.7 -> 14.9  94.4 -> 13.9
+//      256   36.6 -> 12.2  44.1 -> 10.7  33.1 -> 21.5  96.0 -> 19.4
+//     1024   37.2 -> 26.3* 44.1 -> 20.4  68.1          96.6 -> 39.6   (* 1000)
 //     2048   40.5          44.2 -> 28.5  103.6         95.8 -> 59.3
 // Where the last round of 256 x 256 tiles would leave most of the chip idle,
 // its tiles are cut into small ones in a second launch, which costs 8 us here
