@@ -242,15 +242,6 @@ int qh_kv_row_copy(void* k_pool, void* v_pool, const int64_t* src,
  * kv_rows_total bounds cu_k rows: out-of-range rows and pages read zeros.
  */
 size_t qh_attention_workspace_bytes(int n_seqs);
-/*
- * The workspace of a paged call (table != NULL) with which it splits a few
- * queries' keys over more workgroups where that pays; up to about 70 MB. With
- * qh_attention_workspace_bytes(n_seqs), which every call takes, it never
- * splits. A split call's output differs from an unsplit one's by fp32 rounding
- * ahead of the bf16 output. max_q: the longest sequence's queries (a hint).
- */
-size_t qh_attention_paged_workspace_bytes(int n_seqs, int n_queries, int max_q,
-                                          int table_width, int n_q);
 int qh_attention(const void* q, long ldq, int q_rows_total,
                  const int64_t* q_rows, const void* k_pool,
                  const void* v_pool, int pool_pages, const int32_t* table,
@@ -287,8 +278,7 @@ int qh_attention_fp8(const void* q, long ldq, int q_rows_total,
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). The call holds no device memory of its own, so calls may
  * overlap on one GPU. At most 131072 sequences per call (QH_E_ARGUMENT
- * beyond). Output bit-identical to qh_attention_fp8 given
- * qh_attention_workspace_bytes (no split keys).
+ * beyond). Output bit-identical to qh_attention_fp8.
  */
 int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_total,
                              const int64_t* q_rows, const void* k_pool,

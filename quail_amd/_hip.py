@@ -51,7 +51,6 @@ SIGNATURES = {
     "qh_kv_row_scatter": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p],
     "qh_kv_row_copy": [_p, _p, _p, _p, _i, _i, _i, _i, _p],
     "qh_attention_workspace_bytes": [_i],
-    "qh_attention_paged_workspace_bytes": [_i, _i, _i, _i, _i],
     "qh_attention": [_p, _l, _i, _p, _p, _p, _i, _p, _i, _i, _p, _p, _i, _p,
                      _p, _p, _i, _i, _i, _i, _i, _i, _f, _i, _p, _l, _p, _l,
                      _p, _sz, _p],
@@ -79,7 +78,6 @@ SIGNATURES = {
 
 RESTYPES = {
     "qh_last_error": ctypes.c_char_p,
-    "qh_attention_paged_workspace_bytes": ctypes.c_size_t,
     "qh_attention_workspace_bytes": ctypes.c_size_t,
 }
 
@@ -143,11 +141,6 @@ def call(name, *args):
     if status in (QH_E_ARGUMENT, QH_E_UNSUPPORTED, QH_E_WORKSPACE):
         raise ValueError(message)
     raise RuntimeError(message)
-
-
-def paged_workspace_bytes(n_seqs, n_queries, max_q, table_width, n_q) -> int:
-    return int(load().qh_attention_paged_workspace_bytes(int(n_seqs), int(n_queries), int(max_q),
-                                                         int(table_width), int(n_q)))
 
 
 def workspace_bytes(n_seqs: int) -> int:

@@ -72,12 +72,6 @@ struct AttnParams {
   float* out_scales;
   int n_out;
   int ue8m0;
-  // split keys (attn_paged_kernel with SPLIT): per split, unnormalised fp32
-  // output [n_out, n_q, 128] and (running maximum, sum) [n_q, n_out]
-  int splits;
-  int share;  // key tiles of one split
-  float* part_o;
-  float2* part_ml;
 };
 
 // The node-resident tree kernel's two exclusive scans over the segments of
@@ -535,11 +529,7 @@ __device__ __forceinline__ pi32x4 attn_rsrc(const void* base, uint32_t bytes) {
   return (pi32x4){(int)(uint32_t)b, (int)(uint32_t)(b >> 32), (int)bytes, 0x00020000};
 }
 
-// SPLIT: the launch's z index takes one share of the q-tile's key tiles and
-// leaves an unnormalised partial result for attn_combine_kernel. Shares have
-// one size for all sequences: with an equal share of each sequence's own keys,
-// the longest one's workgroups set the launch's time.
-template <bool CAUSAL, bool FP8OUT, bool SPLIT = false>
+template <bool CAUSAL, bool FP8OUT>
 __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
   using namespace pattn;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[NST * STAGE];
@@ -566,23 +556,8 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
   int kv_end = kv_len;
   if (CAUSAL) kv_end = min(kv_len, kv_len - count + min(i0 + BQ, count));
   kv_end = max(kv_end, 0);
-  const int all_tiles = (kv_end + BKV - 1) / BKV;
-  // this workgroup's key tiles: t_begin .. n_tiles
-  int t_begin = 0, n_tiles = all_tiles;
-  if constexpr (SPLIT) {
-    t_begin = (int)blockIdx.z * p.share;
-    // the last share is open-ended (a sum, not a branch: as a branch or a
-    // select of INT_MAX the loop's registers spilled, 72 VGPRs)
-    n_tiles = min(all_tiles, t_begin + ((int)blockIdx.z == p.splits - 1 ? 0x1000000 : p.share));
-  }
+  const int n_tiles = (kv_end + BKV - 1) / BKV;
   const int my_i = i0 + col;
-  if constexpr (SPLIT) {
-    if (t_begin >= n_tiles) {  // past the q-tile's keys: a sum of 0 says so
-      if (my_i < count && half == 0)
-        p.part_ml[((long)blockIdx.z * p.n_q + hq) * p.n_out + q0 + my_i] = make_float2(-1e30f, 0.f);
-      return;
-    }
-  }
   const int lim = CAUSAL ? min(kv_len, kv_len - count + my_i + 1) : kv_len;
 
   // ---- DMA roles ------------------------------------------------------------
@@ -646,19 +621,19 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
                    : "=v"(qraw[st]) : "v"(qoff), "s"(rq), "i"(32 * st) : "memory");
   }
 
-  // ---- prologue: page ids of the first three tiles, DMA of two ---------------
+  // ---- prologue: page ids of tiles 0..2 (scalar), DMA of tiles 0 and 1 -------
   // The page ids are scalar loads through the constant address space: as
   // vector loads behind the Q loads, their vmcnt waits also waited for Q, so
   // the first DMA went out only after a whole Q round trip.
   int pg0 = -1, pg1 = -1, pg2 = -1;
-  if (n_tiles > t_begin) {
+  if (n_tiles > 0) {
     const __attribute__((address_space(4))) int32_t* tab =
         (const __attribute__((address_space(4))) int32_t*)(uintptr_t)(p.table);
-    pg0 = tab[tab_row + min(2 * t_begin + pit, p.table_width - 1)];
-    pg1 = tab[tab_row + min(2 * t_begin + 2 + pit, p.table_width - 1)];
-    pg2 = tab[tab_row + min(2 * t_begin + 4 + pit, p.table_width - 1)];
-    dma_tile(t_begin, pg0, 0);
-    dma_tile(t_begin + 1, pg1, 1);
+    pg0 = tab[tab_row + min(pit, p.table_width - 1)];
+    pg1 = tab[tab_row + min(2 + pit, p.table_width - 1)];
+    pg2 = tab[tab_row + min(4 + pit, p.table_width - 1)];
+    dma_tile(0, pg0, 0);
+    dma_tile(1, pg1, 1);
   }
   asm volatile("s_waitcnt vmcnt(4)" ::: "memory");  // Q and tile 0 landed
   asm volatile("" : "+v"(qraw[0]), "+v"(qraw[1]), "+v"(qraw[2]), "+v"(qraw[3]),
@@ -755,7 +730,7 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
     // are still zero, so the rescale is skipped outright.
     const float traw = tile_row_max(sacc);
     const bool grow = traw > m_thr;
-    if (t == t_begin) {
+    if (t == 0) {
       m_run = grow ? traw * p.scale_log2 : m_run;
       m_thr = (m_run + 8.0f) * inv_scale;
     } else if (__builtin_amdgcn_ballot_w64(grow)) {
@@ -795,7 +770,7 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
     pg_next = ((const __attribute__((address_space(4))) int32_t*)(uintptr_t)(p.table))[
         tab_off(t + 3) / 4];
   };
-  for (int t = t_begin, stage = 0; t < n_tiles; ++t, stage = stage == NST - 1 ? 0 : stage + 1)
+  for (int t = 0, stage = 0; t < n_tiles; ++t, stage = stage == NST - 1 ? 0 : stage + 1)
     step(t, __builtin_amdgcn_readfirstlane(stage));
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no DMA outlives the workgroup
 
@@ -803,20 +778,7 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
   const float l_tot = xor32_sum(l_run);
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   const long qi = q0 + my_i;
-  if constexpr (SPLIT) {
-    if (my_i >= count) return;
-    if (half == 0)
-      p.part_ml[((long)blockIdx.z * p.n_q + hq) * p.n_out + qi] = make_float2(m_run, l_tot);
-    float* po = p.part_o + (((long)blockIdx.z * p.n_out + qi) * p.n_q + hq) * D;
-#pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<float4*>(po + 32 * db + 8 * g + 4 * half) =
-            make_float4(acc_o[db][4 * g], acc_o[db][4 * g + 1], acc_o[db][4 * g + 2],
-                        acc_o[db][4 * g + 3]);
-    return;
-  } else if constexpr (FP8OUT) {
+  if constexpr (FP8OUT) {
     // the bf16 output, quantized per (row, head) 128-wide group exactly as
     // group_quant would quantize it; the group's other 64 values sit in the
     // partner lane (lane ^ 32)
@@ -871,56 +833,6 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
   }
 }
 
-
-// Joins the splits of one (query, head): 32 lanes, four output columns each.
-// Split i's sums are relative to 2^m_i; they are brought to the largest m and
-// added in split order, then the output is written as attn_paged_kernel
-// writes it (bf16, or quantized per head from the bf16 values).
-template <bool FP8OUT>
-__global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
-  constexpr int D = 128;
-  const long item = (long)blockIdx.x * 8 + (threadIdx.x >> 5);
-  const int sub = threadIdx.x & 31;
-  if (item >= (long)p.n_out * p.n_q) return;
-  const int hq = (int)(item % p.n_q);
-  const long qi = item / p.n_q;
-  float m = -1e30f;
-  for (int i = 0; i < p.splits; ++i)
-    m = fmaxf(m, p.part_ml[((long)i * p.n_q + hq) * p.n_out + qi].x);
-  float l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < p.splits; ++i) {
-    const float2 ml = p.part_ml[((long)i * p.n_q + hq) * p.n_out + qi];
-    if (ml.y == 0.f) continue;  // no visible key (its output may not be written)
-    const float w = __builtin_amdgcn_exp2f(ml.x - m);
-    const float4 x = *reinterpret_cast<const float4*>(
-        p.part_o + (((long)i * p.n_out + qi) * p.n_q + hq) * D + 4 * sub);
-    l = __builtin_fmaf(ml.y, w, l);
-    o[0] = __builtin_fmaf(x.x, w, o[0]);
-    o[1] = __builtin_fmaf(x.y, w, o[1]);
-    o[2] = __builtin_fmaf(x.z, w, o[2]);
-    o[3] = __builtin_fmaf(x.w, w, o[3]);
-  }
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
-  float v[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
-  if constexpr (FP8OUT) {
-    round_bf16_pair(v[0], v[1]);
-    round_bf16_pair(v[2], v[3]);
-    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    amax = row_max(amax);
-    amax = fmaxf(amax, __shfl_xor(amax, 16, kWave));
-    const float scale = group_scale(amax, p.ue8m0 != 0);
-    *reinterpret_cast<uint32_t*>(p.out_q + qi * p.ld_out_q + (long)hq * D + 4 * sub) =
-        quant_e4m3_x4(v[0], v[1], v[2], v[3], recip_exact(scale));
-    if (sub == 0) p.out_scales[(long)hq * p.n_out + qi] = scale;
-  } else {
-    *reinterpret_cast<uint2*>(p.out + qi * p.ldo + (long)hq * D + 4 * sub) =
-        make_uint2(f32_to_bf16(v[0]) | (f32_to_bf16(v[1]) << 16),
-                   f32_to_bf16(v[2]) | (f32_to_bf16(v[3]) << 16));
-  }
-  if (p.lse && sub == 0)
-    p.lse[(long)hq * p.lse_stride + qi] =
-        l > 0.f ? (m + log2f(l)) * 0.69314718055994531f : -INFINITY;
-}
 
 // ---------------------------------------------------------------------------
 // Tree attention, fused (the tree path's call A + call B + merge in one pass).
@@ -1826,49 +1738,7 @@ extern "C" size_t qh_attention_workspace_bytes(int n_seqs) {
   return seg_cost_offset(n_seqs) + (size_t)(n_seqs + 1) * sizeof(long long) + 256;
 }
 
-// Into how many shares a paged call's key tiles are split (1: not at all).
-// One q-tile walks its keys one 32-key tile after the other, 0.8 us a tile
-// where its workgroup has a CU to itself (the DMA lead is two tiles), so a few
-// queries over long documents leave most of the chip waiting: 8 documents of
-// 1k-4k tokens x 16 head groups are 128 workgroups. Split, they fill three
-// workgroups on every CU, at the price of the partial results (fp32, a query's
-// whole output per share) and one more launch to join them. Measured, the call
-// with the kernels around it, unsplit / split: 142 / 109 us for those 8
-// documents, 128 / 75 for two, 174 / 158 for 16 (256 workgroups), 46 / 38 for
-// one of 1k tokens under 32 heads. Short documents lose as the workgroups grow
-// in number: 64.6 / 67 us at 16 x 8 workgroups and 1.1k keys, 77 / 88 at
-// 24 x 8, 54 / 58 at 16 x 8 and 0.6k; from 12 keys a workgroup on it pays.
-// Above one workgroup a CU it is within 3% (320 workgroups, 4k keys) or loses
-// (101 / 122 at 1.1k). Two workgroups a CU instead of three: 114 for 109, and
-// 169 for 158. A ring of five tiles at two: 111.
-// The counts are bounds that need no look at device memory: max_q and the
-// table's width only steer the choice.
-static int key_splits(int n_seqs, int n_queries, int max_q, int table_width, int n_q) {
-  if (n_seqs <= 0 || n_queries <= 0 || table_width <= 0) return 1;
-  long tiles = (long)n_queries / attn::BQ + n_seqs;
-  if (max_q > 0) tiles = std::min(tiles, (long)n_seqs * ((max_q + attn::BQ - 1) / attn::BQ));
-  const long groups = std::max(tiles, (long)n_queries / attn::BQ) * (n_q / attn::HPW);
-  const int cus = device_cus();
-  const long keys = (long)table_width * attn::PAGE;
-  if (groups > cus || keys < std::max(512L, 12 * groups)) return 1;
-  const long want = (3L * cus + groups - 1) / groups;
-  return (int)std::max(1L, std::min(std::min(want, 8L), keys / 256));
-}
-static size_t part_ml_bytes(int splits, int n_queries, int n_q) {
-  return ((size_t)splits * n_queries * n_q * sizeof(float2) + 15) & ~(size_t)15;
-}
-static size_t split_bytes(int splits, int n_queries, int n_q) {
-  return splits <= 1 ? 0
-                     : part_ml_bytes(splits, n_queries, n_q) +
-                           (size_t)splits * n_queries * n_q * attn::D * sizeof(float);
-}
-extern "C" size_t qh_attention_paged_workspace_bytes(int n_seqs, int n_queries, int max_q,
-                                                     int table_width, int n_q) {
-  return qh_attention_workspace_bytes(n_seqs) +
-         split_bytes(key_splits(n_seqs, n_queries, max_q, table_width, n_q), n_queries, n_q);
-}
-
-// Shared by qh_attention and qh_attention_fp8: checks, launch.
+// Shared by qh_attention and qh_attention_fp8: checks, tile scan, launch.
 static int attention_launch(const void* q, long ldq, int q_rows_total, const int64_t* q_rows,
                             const void* k_pool, const void* v_pool, int pool_pages,
                             const int32_t* table, int table_width, int page_tokens,
@@ -1947,25 +1817,6 @@ static int attention_launch(const void* q, long ldq, int q_rows_total, const int
   p.ue8m0 = ue8m0;
   const long slots = (long)n_queries / attn::BQ + n_seqs;  // of q-tiles: seq_slot
   dim3 grid((unsigned)slots, (unsigned)(n_q / attn::HPW));
-  const int splits = paged ? key_splits(n_seqs, n_queries, max_q, table_width, n_q) : 1;
-  // a workspace of qh_attention_workspace_bytes never splits, whatever its size
-  if (splits > 1 && workspace_bytes >= qh_attention_workspace_bytes(n_seqs) +
-                                           split_bytes(splits, n_queries, n_q)) {
-    p.splits = splits;
-    const int max_tiles = (table_width * attn::PAGE + pattn::BKV - 1) / pattn::BKV;
-    p.share = (max_tiles + splits - 1) / splits;
-    p.part_ml = (float2*)workspace;
-    p.part_o = (float*)((char*)workspace + part_ml_bytes(splits, n_queries, n_q));
-    grid.z = (unsigned)splits;
-    if (causal) hipLaunchKernelGGL((attn_paged_kernel<true, false, true>), grid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((attn_paged_kernel<false, false, true>), grid, dim3(256), 0, st, p);
-    const int rc = launch_status("attention (split keys)");
-    if (rc) return rc;
-    const dim3 join((unsigned)(((long)n_queries * n_q + 7) / 8));
-    if (fp8) hipLaunchKernelGGL((attn_combine_kernel<true>), join, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL((attn_combine_kernel<false>), join, dim3(256), 0, st, p);
-    return launch_status("attention (joining the splits)");
-  }
   if (paged) {
     if (fp8) {
       if (causal) hipLaunchKernelGGL((attn_paged_kernel<true, true>), grid, dim3(256), 0, st, p);
@@ -2016,8 +1867,8 @@ extern "C" int qh_attention_fp8(const void* q, long ldq, int q_rows_total,
 
 // ---------------------------------------------------------------------------
 // qh_attention_fp8_noalloc: qh_attention_fp8 without a workspace, for callers
-// that cannot allocate. The paged call needs none where it splits no keys; the
-// sequence limit is the one this entry point has always had.
+// that cannot allocate. The paged call needs none; the sequence limit is the
+// one this entry point has always had.
 namespace {
 constexpr int kNoAllocSeqs = 131072;  // sequences one call may carry
 alignas(16) char no_workspace[16];    // stands for a workspace; never dereferenced

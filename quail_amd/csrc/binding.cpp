@@ -316,8 +316,7 @@ PyObject* attention_fp8(PyObject*, PyObject* const* v, Py_ssize_t n) {
   if (d != kGroup) bad_value("one quant group per head needs head_dim 128");
   at::Tensor q = rows_like(q3, n_queries, n_q * d, kE4m3);
   at::Tensor scales = col_major(q3, n_queries, n_q * d);
-  at::Tensor ws = at::empty({(int64_t)qh_attention_paged_workspace_bytes(
-                                (int)n_seqs, (int)n_queries, (int)max_q, (int)table.size(1), (int)n_q)},
+  at::Tensor ws = at::empty({(int64_t)qh_attention_workspace_bytes((int)n_seqs)},
                             q3.options().dtype(at::kByte));
   QH_CALL(qh_attention_fp8, ptr(q3), q3.stride(0), q3.size(0), (const int64_t*)ptr(q_rows),
           ptr(k_pool), ptr(v_pool), k_pool.size(0), (const int32_t*)ptr(table), table.size(1),

@@ -192,9 +192,7 @@ def attention(q3, cu_q, kv_len, *, n_queries, max_q, softmax_scale, causal,
         out = torch.empty((n_queries, n_q, d), dtype=torch.bfloat16, device=dev)
     lse = (torch.empty((n_q, n_queries), dtype=torch.float32, device=dev)
            if want_lse else None)
-    ws_bytes = (_hip.workspace_bytes(n_seqs) if table is None else
-                _hip.paged_workspace_bytes(n_seqs, n_queries, max_q, table.shape[1], n_q))
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    ws = torch.empty(_hip.workspace_bytes(n_seqs), dtype=torch.uint8, device=dev)
     if table is not None:
         pool_pages = k_pool.shape[0]
         table_width = table.shape[1]

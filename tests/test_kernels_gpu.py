@@ -15,7 +15,6 @@ import pytest
 import torch
 
 from oracle import ops as ref
-from quail_amd import _hip
 from quail_amd import kernels as K
 from quail_amd import layout
 
@@ -456,16 +455,13 @@ def test_paged_attention_ignores_unread_rows():
 @pytest.mark.parametrize("n_seqs,prefix,max_suffix,n_q", [(1, 505, 3, 32), (1, 2049, 40, 32),
                                                           (3, 1000, 33, 32), (8, 1600, 24, 64),
                                                           (5, 4100, 70, 64)])
-def test_paged_attention_with_split_keys(n_seqs, prefix, max_suffix, n_q, causal):
-    """A few queries over long documents, whose keys are split over workgroups
-    and joined: against the oracle at the bar of the unsplit call, with a
-    document far shorter than the others (most of its splits are empty), NaN
-    in every arena row no sequence reads, and (not causal) a document of no
-    keys; the fp8 form equals the bf16 form quantized, bit for bit."""
+def test_paged_attention_over_long_documents(n_seqs, prefix, max_suffix, n_q, causal):
+    """A few queries over long documents: against the oracle, with a document
+    far shorter than the others, NaN in every arena row no sequence reads, and
+    (not causal) a document of no keys; the fp8 form equals the bf16 form
+    quantized, bit for bit."""
     case = _paged_case(300 + n_seqs + prefix, n_seqs, prefix, max_suffix, n_q=n_q)
-    T, width = int(case["cu_q"][-1]), case["table"].shape[1]
-    assert (_hip.paged_workspace_bytes(n_seqs, T, case["max_q"], width, n_q)
-            > _hip.workspace_bytes(n_seqs)), "the case does not split"
+    T = int(case["cu_q"][-1])
     if n_seqs > 1:
         case["used"][1] = case["lens"][1] + 17
     if n_seqs > 2 and not causal:
@@ -489,6 +485,80 @@ def test_paged_attention_with_split_keys(n_seqs, prefix, max_suffix, n_q, causal
         q, sc = K.attention_fp8(q_dev, cu, used, ue8m0=ue8m0, **args)
         rq, rs = K.group_quant(out.view(T, -1), ue8m0)
         assert torch.equal(q.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(sc, rs)
+
+
+def _some_sequences(case, seqs):
+    """The sequences `seqs` of a paged case as a call of their own; -1 stands
+    for a sequence of no queries. Returns the call's tensors and the case's
+    query rows it covers."""
+    cu = case["cu_q"].tolist()
+    rows = [torch.arange(cu[s], cu[s + 1]) if s >= 0 else torch.arange(0) for s in seqs]
+    at = torch.tensor([max(s, 0) for s in seqs])
+    lens = torch.tensor([len(r) for r in rows])
+    part = dict(case, table=case["table"][at], used=case["used"][at],
+                cu_q=torch.cat([torch.zeros(1, dtype=torch.int32), lens.cumsum(0).to(torch.int32)]),
+                max_q=int(lens.max()))
+    rows = torch.cat(rows)
+    part["q"] = case["q"][rows]
+    return part, rows
+
+
+@pytest.mark.parametrize("causal,gathered", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("n_seqs,prefix,max_suffix,n_q", [(40, 505, 3, 32), (24, 2049, 40, 32),
+                                                          (24, 1600, 24, 64), (9, 1100, 70, 64)])
+def test_paged_attention_bits_do_not_depend_on_the_chunk(n_seqs, prefix, max_suffix, n_q, causal,
+                                                         gathered):
+    """A query's output is one walk over its own keys, whatever else is in the
+    call: one sequence alone, a few of them, and a few among sequences of no
+    queries (first, last, and two in a row) give the bits that the call of all
+    of them gives, in bf16, in the log-sum-exp and in the fp8 form, with q in
+    place or gathered."""
+    case = _paged_case(300 + n_seqs + prefix, n_seqs, prefix, max_suffix, n_q=n_q)
+    case["used"][1] = case["lens"][1] + 17   # a document far shorter than the others
+    kp = layout.k_pool_from_rows(case["k_rows"]).to(DEV)
+    vp = layout.v_pool_from_rows(case["v_rows"]).to(DEV)
+
+    def call(part):
+        q, rows = part["q"].to(DEV), None
+        T = q.shape[0]
+        if gathered:
+            rows = torch.randperm(T + 30, generator=_gen(5))[:T].to(DEV)
+            q = torch.zeros(T + 30, n_q, 128, dtype=torch.bfloat16, device=DEV).index_copy(0, rows, q)
+        args = dict(n_queries=T, max_q=part["max_q"], softmax_scale=1 / math.sqrt(128),
+                    causal=causal, k_pool=kp, v_pool=vp, table=part["table"].to(DEV), q_rows=rows,
+                    n_kv=case["n_kv"])
+        cu, used = part["cu_q"].to(DEV), part["used"].to(DEV)
+        out, lse = K.attention(q, cu, used, want_lse=True, **args)
+        q8, s8 = K.attention_fp8(q, cu, used, **args)
+        return [out.view(torch.int16), lse.t().contiguous().view(torch.int32),
+                q8.view(torch.uint8), s8.contiguous().view(torch.int32)]
+
+    full = call(case)
+    for seqs in ([0], [1], [n_seqs - 1], [2, 5, 3], list(range(8)),
+                 [-1, 0, -1, -1, 4, 1, -1], [-1] + list(range(n_seqs)) + [-1]):
+        part, rows = _some_sequences(case, seqs)
+        for i, (x, y) in enumerate(zip(call(part), full)):
+            assert torch.equal(x, y[rows.to(DEV)]), (seqs, i)
+
+
+@pytest.mark.parametrize("n_seqs,prefix", [(2, 700), (12, 90)])
+def test_paged_attention_leaves_rows_of_no_sequence_alone(n_seqs, prefix):
+    """n_queries is a bound: where the sequences cover a part of the query rows
+    only (cu_q[0] > 0, cu_q[n] < n_queries), the call writes that part, with the
+    bits of the call of all of them, and leaves the rest of a caller's output."""
+    case = _paged_case(500 + n_seqs, n_seqs + 2, prefix, 40)
+    cu, T = case["cu_q"], int(case["cu_q"][-1])
+    args = dict(n_queries=T, max_q=case["max_q"], softmax_scale=1 / math.sqrt(128), causal=True,
+                k_pool=layout.k_pool_from_rows(case["k_rows"]).to(DEV),
+                v_pool=layout.v_pool_from_rows(case["v_rows"]).to(DEV), n_kv=case["n_kv"])
+    q = case["q"].to(DEV)
+    full, _ = K.attention(q, cu.to(DEV), case["used"].to(DEV), table=case["table"].to(DEV), **args)
+    out = torch.full_like(full, 7.0)
+    K.attention(q, cu[1:-1].to(DEV), case["used"][1:-1].to(DEV), table=case["table"][1:-1].to(DEV),
+                out=out, **args)
+    lo, hi = int(cu[1]), int(cu[-2])
+    assert torch.equal(out[lo:hi].view(torch.int16), full[lo:hi].view(torch.int16))
+    assert (out[:lo] == 7).all() and (out[hi:] == 7).all()
 
 
 @pytest.mark.parametrize("causal,gathered", [(True, False), (False, True)])
