@@ -44,7 +44,12 @@ struct Shape {
   static constexpr int NB = EPI == kSiluQuant || (EPI == kQkvRope && BR == 256 && NR == 4) ? 2 : 1;
   static constexpr int SBROW = 4 * MAX_NK;
   static constexpr int SBROWS = BR == 256 ? 2 : 1;
-  static constexpr int LDS_LOOP = NS * STAGE + SBROWS * SBROW;
+  // The last step reads ahead like the others, into registers that nobody uses:
+  // up to scale KU ceil(nk / KU) + KU - 1 of a row, which for nk = 253 .. 255 and
+  // four blocks a step lies past the last row. The pad keeps it inside.
+  static constexpr int SB_END = 4 * ((MAX_NK - 1 + KU - 1) / KU * KU + KU);
+  static constexpr int SB_PAD = SB_END > SBROW ? SB_END - SBROW : 0;
+  static constexpr int LDS_LOOP = NS * STAGE + SBROWS * SBROW + SB_PAD;
   static constexpr int LDS_EPI = BM * OROW + EXTRA;
   static constexpr int LDS = LDS_LOOP > LDS_EPI ? LDS_LOOP : LDS_EPI;
   static_assert(BM <= 64 || (BM <= 128 && NW % 2 == 0), "the scale DMA covers the tile's tokens");
@@ -52,6 +57,7 @@ struct Shape {
   static_assert(EPI == kStoreBf16 || BR == 256 || (EPI == kQkvRope && BR == 128),
                 "a fused epilogue needs whole heads, or the gate and up rows of a group");
   static_assert(LDS <= 160 * 1024, "LDS");
+  static_assert(NS * STAGE + (SBROWS - 1) * SBROW + SB_END <= LDS, "the read ahead's last scale");
 };
 
 // f(0) .. f(N - 1) with compile-time arguments: fragment arrays indexed by an

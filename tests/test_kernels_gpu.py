@@ -304,17 +304,13 @@ def _head_rows(sa, m):
     return out
 
 
-@pytest.mark.parametrize("ue8m0", [False, True])
-@pytest.mark.parametrize("epilogue,Kd", [("store", 128), ("store", 1152), ("store", 4224),
-                                         ("silu", 128), ("silu", 1152), ("qkv", 128),
-                                         ("qkv", 1152), ("qkv", 2560)])
-def test_fp8_gemm_bits_do_not_depend_on_the_chunk_size(epilogue, Kd, ue8m0):
-    """A token's output has one order of products and promotions whatever
-    tiling its chunk takes: the first m rows of an 18,000-token call (256 x
-    256 tiles) equal an m-token call bit for bit, for every epilogue, odd,
-    even and single K blocks, and both scale modes; arena pages included."""
-    n_q, n_kv, M = 32, 8, 18000
-    N = {"store": 2560, "silu": 5120, "qkv": (n_q + 2 * n_kv) * 128}[epilogue]
+def _gemm_calls(epilogue, M, Kd, ue8m0, heads=(32, 8), N=None):
+    """call(m, blocks): the GEMM with `epilogue` over the first m of M tokens,
+    its outputs as integers (token rows first). blocks > Kd / 128 appends K
+    blocks of zeros, which add +0 to every sum: the same bits. K = 256 blocks
+    and more take 256 x 256 tiles only, whatever m."""
+    n_q, n_kv = heads
+    N = N or {"store": 2560, "silu": 5120, "qkv": (n_q + 2 * n_kv) * 128}[epilogue]
     a, sa, w, sw = _gemm_inputs(21, M, N, Kd, DEV)
     if ue8m0:
         sa = sa.clone(memory_format=torch.preserve_format)
@@ -328,13 +324,23 @@ def test_fp8_gemm_bits_do_not_depend_on_the_chunk_size(epilogue, Kd, ue8m0):
     pages = M // 16 + 2
     dst = (torch.arange(M) + 7).to(DEV)   # runs that start and end inside a page
 
-    def call(m):
-        args = (a[:m], _head_rows(sa, m), w, sw)
+    def operands(m, blocks):
+        if blocks is None:
+            return a[:m], _head_rows(sa, m), w, sw
+        pad = blocks * 128 - Kd
+        scales = K.col_major_scales(m, blocks * 128, DEV).fill_(1.0)
+        scales[:, :Kd // 128] = sa[:m]
+        zeros = lambda x: torch.nn.functional.pad(x.view(torch.uint8), (0, pad))  # noqa: E731
+        return (zeros(a[:m]).view(a.dtype), scales, zeros(w).view(w.dtype),
+                torch.nn.functional.pad(sw, (0, pad // 128), value=1.0))
+
+    def call(m, blocks=None):
+        args = operands(m, blocks)
         if epilogue == "store":
-            return [K.fp8_gemm_nt(*args, ue8m0_scales=ue8m0)]
+            return [K.fp8_gemm_nt(*args, ue8m0_scales=ue8m0).view(torch.int16)]
         if epilogue == "silu":
             q, s = K.fp8_gemm_silu_quant(*args, ue8m0, ue8m0_scales=ue8m0)
-            return [q.view(torch.uint8), s.contiguous()]
+            return [q.view(torch.uint8), s.contiguous().view(torch.int32)]
         rows = K.fp8_gemm_qkv_rope(*args, pos[:m].contiguous(), *rope, ue8m0_scales=ue8m0)
         kp = torch.zeros(pages, n_kv, 16, 128, dtype=torch.bfloat16, device=DEV)
         vp = torch.zeros(pages, n_kv, 128, 16, dtype=torch.bfloat16, device=DEV)
@@ -344,14 +350,43 @@ def test_fp8_gemm_bits_do_not_depend_on_the_chunk_size(epilogue, Kd, ue8m0):
         k_rows, v_rows = layout.k_rows(kp), layout.v_rows(vp)
         untouched = torch.cat([k_rows[:7], k_rows[m + 7:], v_rows[:7], v_rows[m + 7:]])
         assert not untouched.view(torch.int16).any()
-        return list(rows) + [k_rows[7:m + 7], v_rows[7:m + 7]]
+        outs = list(rows) + [k_rows[7:m + 7], v_rows[7:m + 7]]
+        return [x.contiguous().view(torch.int16) for x in outs]
 
+    return call
+
+
+@pytest.mark.parametrize("ue8m0", [False, True])
+@pytest.mark.parametrize("epilogue,Kd", [("store", 128), ("store", 256), ("store", 384),
+                                         ("store", 512), ("store", 1152), ("store", 4096),
+                                         ("store", 4224), ("silu", 128), ("silu", 256),
+                                         ("silu", 1152), ("qkv", 128), ("qkv", 256),
+                                         ("qkv", 1152), ("qkv", 2560)])
+def test_fp8_gemm_bits_do_not_depend_on_the_chunk_size(epilogue, Kd, ue8m0):
+    """A token's output has one order of products and promotions whatever
+    tiling its chunk takes: the first m rows of an 18,000-token call (mostly
+    256 x 256 tiles) equal an m-token call bit for bit, for every epilogue,
+    both scale modes, a single K block and every remainder of the tilings that
+    take four at a time; arena pages included."""
+    M = 18000
+    call = _gemm_calls(epilogue, M, Kd, ue8m0)
     full = call(M)
     for m in TILING_SIZES:
         for i, (x, y) in enumerate(zip(call(m), full)):
-            bits = torch.uint8 if x.dtype == torch.uint8 else (
-                torch.int32 if x.dtype == torch.float32 else torch.int16)
-            assert torch.equal(x.contiguous().view(bits), y[:m].contiguous().view(bits)), (m, i)
+            assert torch.equal(x, y[:m]), (m, i)
+
+
+@pytest.mark.parametrize("ue8m0", [False, True])
+@pytest.mark.parametrize("epilogue", ["store", "silu", "qkv"])
+@pytest.mark.parametrize("nk", [253, 254, 255])
+def test_fp8_gemm_small_tilings_at_their_longest_K(nk, epilogue, ue8m0):
+    """253 to 255 K blocks are the most that the small tilings' LDS holds the
+    weight scales of, and their last step reads ahead past them; one block
+    more takes 256 x 256 tiles, here with blocks of zeros as the reference."""
+    call = _gemm_calls(epilogue, 700, 128 * nk, ue8m0, heads=(8, 2), N=None if epilogue == "qkv" else 512)
+    for m in (1, 17, 33, 150, 700):
+        for i, (x, y) in enumerate(zip(call(m), call(m, 256))):
+            assert torch.equal(x, y), (m, i)
 
 
 def test_fp8_gemm_silu_quant_oracle():
