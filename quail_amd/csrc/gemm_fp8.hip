@@ -48,6 +48,8 @@
 #include <type_traits>
 #include <utility>
 
+#include "gemm_plan.h"
+
 namespace qh {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -56,17 +58,12 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 namespace gemm {
-constexpr int BM = 256;         // tile tokens
-constexpr int BR = 256;         // tile weight rows
-constexpr int BK = 128;         // K block: one MFMA, one scale block
 constexpr int NS = 4;           // weight stages in LDS
 constexpr int PA = 2;           // scale blocks in flight ahead
 constexpr int STAGE = BR * BK;  // 32 KiB
 constexpr int A_WAVE = 32 * BK; // 4 KiB: a wave's 32 tokens of one K block
 constexpr int LOADS = 12;       // vector-memory loads per wave per step
 constexpr int XCDS = 8;
-constexpr int GROUP_M = 4;      // tile rows per column sweep (see launch_gemm)
-enum { kStoreBf16 = 0, kSiluQuant = 1, kQkvRope = 2 };
 }  // namespace gemm
 
 // The qkv projection's fused epilogue (kQkvRope): per-head q/k RMSNorm +
@@ -119,16 +116,6 @@ __device__ __forceinline__ i32x4 buffer_rsrc(const void* base, uint32_t bytes) {
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
-// Tile t of tiles_m x tiles_n in tile order: group_m tile rows per column sweep.
-__device__ __forceinline__ void tile_at(int t, int group_m, int tiles_m, int tiles_n, int& tm,
-                                        int& tn) {
-  const int in_group = group_m * tiles_n;
-  const int first_m = (t / in_group) * group_m;
-  const int gsize = min(tiles_m - first_m, group_m);
-  tm = first_m + (t % in_group) % gsize;
-  tn = (t % in_group) / gsize;
 }
 
 // silu(gate) * up of one GEMM output pair, with both rounded to bf16 first:
@@ -810,7 +797,7 @@ namespace qh {
 // the same bits.
 template <int EPI, bool HW>
 static int dispatch_gemm(const GemmArgs& a, qh_stream_t stream, const char* what) {
-  const gemm_small::Plan plan = gemm_small::choose(EPI, a.M, a.N, a.K);
+  const gemm_small::Plan plan = gemm_small::choose(EPI, a.M, a.N, a.K, device_cus());
   GemmArgs part = a;
   part.ld_sa = a.M;
   part.tile0 = 0;

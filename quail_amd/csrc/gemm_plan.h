@@ -1,0 +1,145 @@
+// How a call of the fp8 GEMM is cut into tiles: plain C++, so that the CPU tests
+// compile it as it stands.
+#pragma once
+
+#include <algorithm>
+
+#ifdef __HIPCC__
+#define QH_HD __host__ __device__ __forceinline__
+#else
+#define QH_HD inline
+#endif
+
+namespace qh {
+
+namespace gemm {
+constexpr int BM = 256;     // tile tokens
+constexpr int BR = 256;     // tile weight rows
+constexpr int BK = 128;     // K block: one MFMA, one scale block
+constexpr int GROUP_M = 4;  // tile rows per column sweep (see launch_gemm)
+enum { kStoreBf16 = 0, kSiluQuant = 1, kQkvRope = 2 };
+}  // namespace gemm
+
+// Tile t of tiles_m x tiles_n in tile order: group_m tile rows per column sweep.
+QH_HD void tile_at(int t, int group_m, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int in_group = group_m * tiles_n;
+  const int first_m = (t / in_group) * group_m;
+  const int gsize = tiles_m - first_m < group_m ? tiles_m - first_m : group_m;
+  tm = first_m + (t % in_group) % gsize;
+  tn = (t % in_group) / gsize;
+}
+
+namespace gemm_small {
+
+constexpr int MAX_NK = 256;  // K blocks whose weight scales a small tiling's LDS rows hold
+
+// A tiling's cost model: tiles in rounds of one per CU, `fixed` us plus per K
+// block `first` us for the first round and `more` us for each further one
+// (shorter where two workgroups share a CU, longer where a full chip runs at a
+// lower clock). Fitted over the Qwen3-4B and Qwen3-32B projections at 1 to
+// 40,000 tokens (248 sizes, every tiling timed at each, one MI355X).
+struct Tiling {
+  int rows, tokens;
+  float fixed, first, more;
+};
+constexpr Tiling kLarge[3] = {{256, 256, 2.7f, 1.288f, 1.784f},    // kStoreBf16
+                              {256, 256, 0.0f, 1.726f, 1.822f},    // kSiluQuant
+                              {256, 256, 11.9f, 1.214f, 1.975f}};  // kQkvRope
+constexpr int kTilings[3] = {7, 4, 5};
+constexpr Tiling kSmall[3][7] = {
+    {{32, 16, 4.1f, 0.104f, 0.132f},
+     {64, 16, 2.6f, 0.161f, 0.162f},
+     {64, 32, 2.8f, 0.186f, 0.193f},
+     {64, 64, 2.4f, 0.245f, 0.268f},
+     {128, 64, 0.5f, 0.408f, 0.326f},
+     {128, 128, 3.1f, 0.498f, 0.629f},
+     {256, 128, 2.6f, 0.767f, 1.001f}},
+    {{256, 16, 0.f, 0.704f, 0.568f},
+     {256, 32, 0.f, 0.797f, 0.682f},
+     {256, 64, 0.f, 0.900f, 0.780f},
+     {256, 128, 0.f, 1.155f, 1.125f}},
+    {{128, 16, 4.3f, 0.236f, 0.249f},
+     {128, 32, 4.1f, 0.278f, 0.256f},
+     {128, 64, 5.5f, 0.314f, 0.469f},
+     {128, 128, 7.5f, 0.430f, 0.771f},
+     {256, 128, 10.2f, 0.672f, 1.249f}}};
+
+// How a chunk is tiled: the first `large` 256 x 256 tiles, in tile order, as
+// such, the rest, if any, on tiling `small` (an index into kSmall[epi]).
+struct Plan {
+  int large, small;
+};
+
+static int all_tiles(int M, int N) {
+  return ((M + gemm::BM - 1) / gemm::BM) * (N / gemm::BR);
+}
+
+// How many of the 256 x 256 tiles from tile `from` on are in the last tile row.
+static int last_row_tiles(int from, int M, int N) {
+  const int tiles_m = (M + gemm::BM - 1) / gemm::BM, tiles_n = N / gemm::BR;
+  const int first_m = (tiles_m - 1) / gemm::GROUP_M * gemm::GROUP_M;  // of the last group
+  return tiles_n - std::max(0, from - first_m * tiles_n) / (tiles_m - first_m);
+}
+
+// The plan with the lowest cost, the small tilings' taken 10 % up (so that no
+// size of the fit runs slower than on 256 x 256 tiles alone; without it eight
+// did, by up to 9 %). With one tiling for all tokens the choice costs 0.02 %
+// on average and 2 % at most against the best measured one. Against 256 x 256
+// tiles alone (us, Qwen3-4B):
+//   tokens   qkv           o             gate_up       down
+//        1   33.4 ->  8.8  43.0 ->  6.9  31.9 -> 12.4  93.0 -> 11.3
+//       64   34.0 ->  9.3  42.9 ->  8.3  32.7 -> 14.9  94.4 -> 13.9
+//      256   36.6 -> 12.2  44.1 -> 10.7  33.1 -> 21.5  96.0 -> 19.4
+//     1024   37.2 -> 26.3* 44.1 -> 20.4  68.1          96.6 -> 39.6   (* 1000)
+//     2048   40.5          44.2 -> 28.5  103.6         95.8 -> 59.3
+// Where the last round of 256 x 256 tiles would leave most of the chip idle,
+// its tiles are cut into small ones in a second launch, which costs 8 us here
+// (its start, and a first round on cold LDS; with 4 two sizes ran up to 4 %
+// slower than unsplit). Tiles and not whole tile rows: gate_up has 76 tiles a
+// row. Measured (us, 256 x 256 tiles alone -> so): gate_up at 1,157 tokens, 380
+// tiles on 256 CUs, 69.3 -> 63.5, at 900 72 -> 58; o at 7,200 tokens, 290 tiles,
+// 99 -> 81; down 225 -> 185, at 14,000 358 -> 328; qkv at 3,000 75 -> 59;
+// Qwen3-32B at 4,000 tokens o 184 -> 154, down 578 -> 482.
+static Plan choose(int epi, int M, int N, int K, int cus) {
+  const int all = all_tiles(M, N);
+  const int nk = K / gemm::BK;
+  if (nk >= MAX_NK) return {all, 0};  // the scale rows in LDS hold fewer blocks
+  auto cost = [&](const Tiling& t, long tiles) {
+    const long rounds = (tiles + cus - 1) / cus;
+    return t.fixed + (float)nk * (t.first + t.more * (float)(rounds - 1));
+  };
+  // tiles of tiling t in the 256 x 256 tiles from `from` on
+  auto pieces = [&](const Tiling& t, int from) {
+    const int last = last_row_tiles(from, M, N);
+    const int tokens = M - (M - 1) / gemm::BM * gemm::BM;  // of the last tile row
+    return ((long)(all - from - last) * (gemm::BM / t.tokens) +
+            (long)last * ((tokens + t.tokens - 1) / t.tokens)) * (gemm::BR / t.rows);
+  };
+  Plan best = {all, 0};
+  float least = cost(kLarge[epi], all);
+  auto with_small = [&](int large) {
+    const float ahead = large > 0 ? cost(kLarge[epi], large) + 8.f : 0.f;
+    for (int i = 0; i < kTilings[epi]; ++i) {
+      const float c = ahead + 1.10f * cost(kSmall[epi][i], pieces(kSmall[epi][i], large));
+      if (c < least) {
+        least = c;
+        best = {large, i};
+      }
+    }
+  };
+  with_small(0);
+  // whole rounds of 256 x 256 tiles, all but the last one or two (gate_up: the
+  // last; one more round in small tiles, 128 tokens at best, measured 1 % slower
+  // than unsplit at 6,000 tokens and never best)
+  const int rounds = all / cus;
+  for (int r = rounds; r >= 1 && r >= rounds - (epi == gemm::kSiluQuant ? 0 : 1); --r) {
+    // qkv past two rounds: the split measured -3 to +5 % (its long epilogues
+    // overlap the next tile's start in the persistent kernel)
+    if (epi == gemm::kQkvRope && r > 2) continue;
+    if (r * cus < all) with_small(r * cus);
+  }
+  return best;
+}
+
+}  // namespace gemm_small
+}  // namespace qh
