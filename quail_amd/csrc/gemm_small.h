@@ -93,19 +93,13 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
   // or the pieces, neighbours in launch order, of 256 x 256 tiles tile0 and up ----
   int tm, tn;
   {
-    constexpr int CM = gemm::BM / S::BM, CN = gemm::BR / S::BR;  // pieces of a 256 x 256 tile
     const int n = (int)gridDim.x, per = n / gemm::XCDS;
     int t = (int)blockIdx.x;
     if (t < per * gemm::XCDS) t = (t % gemm::XCDS) * per + t / gemm::XCDS;
-    if (p.tile0 == 0) {
+    if (p.tile0 == 0)
       tile_at(t, p.group_m, (M + S::BM - 1) / S::BM, p.N / S::BR, tm, tn);
-    } else {
-      tile_at(p.tile0 + t / (CM * CN), gemm::GROUP_M, (M + gemm::BM - 1) / gemm::BM,
-              p.N / gemm::BR, tm, tn);
-      tm = tm * CM + t % CM;
-      tn = tn * CN + t % (CM * CN) / CM;
-      if (tm * S::BM >= M) return;  // past the last token
-    }
+    else
+      Pieces(p.tile0, M, p.N, S::BM, S::BR).at(t, tm, tn);
   }
   const int m0 = tm * S::BM;
 
@@ -549,9 +543,8 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
 template <int EPI, bool HW, int NR, int WT, int RT, int TM, int KU, int NS, int OCC>
 static int launch(GemmArgs a, qh_stream_t stream, const char* what) {
   using S = Shape<EPI, NR, WT, RT, TM, KU, NS>;
-  const int tiles = a.tile0 == 0
-                        ? ((a.M + S::BM - 1) / S::BM) * (a.N / S::BR)
-                        : (a.tiles - a.tile0) * (gemm::BM / S::BM) * (gemm::BR / S::BR);
+  const int tiles = a.tile0 == 0 ? ((a.M + S::BM - 1) / S::BM) * (a.N / S::BR)
+                                 : (int)Pieces(a.tile0, a.M, a.N, S::BM, S::BR).count();
   a.group_m = 8;
   hipLaunchKernelGGL((fp8_gemm_small_kernel<EPI, HW, NR, WT, RT, TM, KU, NS, OCC>), dim3(tiles),
                      dim3(64 * S::NW), 0, (hipStream_t)stream, a);
