@@ -6,6 +6,8 @@
 // on its own, as in the reference's op-by-op fp32 expressions.
 #include "common.h"
 
+#include <type_traits>
+
 namespace qh {
 
 // ---------------------------------------------------------------------------
@@ -555,13 +557,19 @@ __global__ __launch_bounds__(256) void final_norm_kernel(
 
 // ---------------------------------------------------------------------------
 // Answer readout: per row, bf16 scores against the retained answer rows,
-// strict TRUE > FALSE compare (readout.py:45-49, :70-79). One workgroup per
-// row, wave w takes answers w, w + 4, .. two at a time: with one wave per row
-// the answers' dot products (each 2 H loads and a 64-lane sum) ran one after
-// the other, and 409 rows of 2560 against 8 answers took 12.2 us of which the
-// bytes need 1; now 4.6.
-constexpr int kAnswerWaves = 4;
+// strict TRUE > FALSE compare (readout.py:45-49, :70-79). W waves per row: wave
+// w takes answers w, w + W, .. two at a time, a last odd one alone.
+// With one wave per row the answers' dot products (each 2 H loads and a 64-lane
+// sum) run one after the other (409 rows of 2560 against 8 answers 11.4 us, now
+// 4.3); with more waves than pairs of answers the others find no answer, and a
+// full chip of rows waits for them. Measured (us, 1 / 2 / 4 waves a row): 7,200 rows
+// of 2560 against 1 answer 6.0 / 7.2 / 11.5, 2 answers 7.3 / 7.9 / 12.0, 4 answers
+// 11.2 / 10.3 / 13.4, 8 answers 19.2 / 17.5 / 17.5; 16,384 rows of 5120 against 2
+// answers 25.9 / 27.0 / 41.0, 4 answers 47.8 / 37.1 / 46.9, 8 answers 92.8 / 72.7 /
+// 69.2. Below 2,000 rows fewer waves than pairs only lengthen the chain.
+constexpr int kAnswerWaves = 4;  // of a workgroup
 
+template <int W>
 __global__ __launch_bounds__(64 * kAnswerWaves) void answer_bits_kernel(
     const uint16_t* __restrict__ normed, int R, int H,
     const uint16_t* __restrict__ w_ans, int n_ans,
@@ -569,45 +577,52 @@ __global__ __launch_bounds__(64 * kAnswerWaves) void answer_bits_kernel(
     float* __restrict__ margin, uint16_t* __restrict__ best_true,
     uint16_t* __restrict__ best_false) {
   __shared__ float best[kAnswerWaves][2];
-  const int i = blockIdx.x;
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const uint16_t* row = normed + (long)i * H;
+  const int i = blockIdx.x * (kAnswerWaves / W) + wave / W;
   float best_t = -INFINITY, best_f = -INFINITY;
-  auto take = [&](int a, float acc) __attribute__((always_inline)) {
-    const float score = round_bf16(wave_sum(acc));
-    if (is_true[a]) best_t = fmaxf(best_t, score);
-    else best_f = fmaxf(best_f, score);
-  };
-  for (int a = wave; a < n_ans; a += 2 * kAnswerWaves) {
-    const int b = a + kAnswerWaves;
-    const uint16_t* wa = w_ans + (long)a * H;
-    const uint16_t* wb = w_ans + (long)(b < n_ans ? b : a) * H;
-    float acc_a = 0.f, acc_b = 0.f;
+  if (i < R) {
+    const uint16_t* row = normed + (long)i * H;
+    auto score = [&](int a, float acc) __attribute__((always_inline)) {
+      const float x = round_bf16(wave_sum(acc));
+      if (is_true[a]) best_t = fmaxf(best_t, x);
+      else best_f = fmaxf(best_f, x);
+    };
+    auto take = [&](int a, int b, auto pair_c) __attribute__((always_inline)) {
+      constexpr bool PAIR = decltype(pair_c)::value;
+      const uint16_t* wa = w_ans + (long)a * H;
+      const uint16_t* wb = w_ans + (long)b * H;
+      float acc_a = 0.f, acc_b = 0.f;
 #pragma unroll 5
-    for (int c = lane * 8; c < H; c += 512) {
-      const bf16x8 nv = load8(row + c);
-      const bf16x8 va = load8(wa + c);
-      const bf16x8 vb = load8(wb + c);
+      for (int c = lane * 8; c < H; c += 512) {
+        const bf16x8 nv = load8(row + c);
+        const bf16x8 va = load8(wa + c);
+        bf16x8 vb;
+        if constexpr (PAIR) vb = load8(wb + c);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        acc_a += nv.get(e) * va.get(e);
-        acc_b += nv.get(e) * vb.get(e);
+        for (int e = 0; e < 8; ++e) {
+          acc_a += nv.get(e) * va.get(e);
+          if constexpr (PAIR) acc_b += nv.get(e) * vb.get(e);
+        }
       }
+      score(a, acc_a);
+      if constexpr (PAIR) score(b, acc_b);
+    };
+    for (int a = wave % W; a < n_ans; a += 2 * W) {
+      if (a + W < n_ans) take(a, a + W, std::true_type{});
+      else take(a, a, std::false_type{});
     }
-    take(a, acc_a);
-    if (b < n_ans) take(b, acc_b);
   }
   if (lane == 0) {
     best[wave][0] = best_t;
     best[wave][1] = best_f;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (lane == 0 && wave % W == 0 && i < R) {
 #pragma unroll
-    for (int k = 1; k < kAnswerWaves; ++k) {
-      best_t = fmaxf(best_t, best[k][0]);
-      best_f = fmaxf(best_f, best[k][1]);
+    for (int k = 1; k < W; ++k) {
+      best_t = fmaxf(best_t, best[wave + k][0]);
+      best_f = fmaxf(best_f, best[wave + k][1]);
     }
     if (bits) bits[i] = best_t > best_f ? 1 : 0;
     if (margin) margin[i] = best_t - best_f;
@@ -849,17 +864,30 @@ extern "C" int qh_fused_add_rms_norm(void* hidden, void* residual, int R, int H,
                            "fused_add_rms_norm");
 }
 
+static int launch_answers(const void* normed, int R, int H, const void* w_ans, int n_ans,
+                          const uint8_t* is_true, uint8_t* bits, float* margin, void* best_true,
+                          void* best_false, qh_stream_t stream, const char* what) {
+  auto run = [&](auto kern, int waves) {
+    hipLaunchKernelGGL(kern, dim3(blocks_for(R, kAnswerWaves / waves)), dim3(64 * kAnswerWaves), 0,
+                       (hipStream_t)stream, (const uint16_t*)normed, R, H, (const uint16_t*)w_ans,
+                       n_ans, is_true, bits, margin, (uint16_t*)best_true, (uint16_t*)best_false);
+  };
+  // one wave per pair of answers, up to four (the figures are at the kernel);
+  // from 2^24 rows on one, as a launch holds fewer than 2^32 threads
+  if (n_ans <= 2 || R >= 1 << 24) run(answer_bits_kernel<1>, 1);
+  else if (n_ans <= 4) run(answer_bits_kernel<2>, 2);
+  else run(answer_bits_kernel<4>, 4);
+  return launch_status(what);
+}
+
 extern "C" int qh_answer_bits(const void* normed, int R, int H, const void* w_ans,
                               int n_ans, const uint8_t* is_true, uint8_t* bits,
                               float* margin, qh_stream_t stream) {
   QH_REQUIRE(R >= 0 && H > 0 && H % 8 == 0 && n_ans > 0, "answer_bits: geometry");
   if (R == 0) return QH_OK;
   QH_REQUIRE(normed && w_ans && is_true && bits, "answer_bits: null pointer");
-  hipLaunchKernelGGL(answer_bits_kernel, dim3(R), dim3(64 * kAnswerWaves), 0,
-                     (hipStream_t)stream, (const uint16_t*)normed, R, H,
-                     (const uint16_t*)w_ans, n_ans, is_true, bits, margin,
-                     (uint16_t*)nullptr, (uint16_t*)nullptr);
-  return launch_status("answer_bits");
+  return launch_answers(normed, R, H, w_ans, n_ans, is_true, bits, margin, nullptr, nullptr, stream,
+                        "answer_bits");
 }
 
 extern "C" int qh_e4m3_encode(const float* x, long n, uint8_t* out, qh_stream_t stream) {
@@ -879,9 +907,6 @@ extern "C" int qh_answer_logits(const void* normed, int R, int H, const void* w_
   if (R == 0) return QH_OK;
   QH_REQUIRE(normed && w_ans && is_true && best_true && best_false,
              "answer_logits: null pointer");
-  hipLaunchKernelGGL(answer_bits_kernel, dim3(R), dim3(64 * kAnswerWaves), 0,
-                     (hipStream_t)stream, (const uint16_t*)normed, R, H,
-                     (const uint16_t*)w_ans, n_ans, is_true, (uint8_t*)nullptr,
-                     (float*)nullptr, (uint16_t*)best_true, (uint16_t*)best_false);
-  return launch_status("answer_logits");
+  return launch_answers(normed, R, H, w_ans, n_ans, is_true, nullptr, nullptr, best_true, best_false,
+                        stream, "answer_logits");
 }

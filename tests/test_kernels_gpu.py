@@ -859,11 +859,13 @@ def test_gather_final_norm_and_answer_bits():
 
 
 @pytest.mark.parametrize("H", [8, 520, 2560, 2568, 5120, 5128, 8192])
-@pytest.mark.parametrize("R,n_ans", [(1, 1), (5, 2), (5, 9), (409, 8)])
+@pytest.mark.parametrize("R,n_ans", [(1, 1), (5, 2), (7, 3), (402, 4), (3, 5), (5, 9), (409, 8),
+                                     (6, 17)])
 def test_final_norm_and_readout_at_every_width(R, n_ans, H):
     """The register-held norm (H up to 2560 and 5120, partial last vectors) and
-    the two-pass one above it, gathered and in place, and the scores of 1 to 9
-    answers over the workgroup's waves, against the oracle."""
+    the two-pass one above it, gathered and in place, and the scores of 1 to 17
+    answers over one, two and four waves a row (whole and partly filled
+    workgroups), against the oracle."""
     g = _gen(61 + R + H)
     hidden = torch.randn(R + 3, H, generator=g).to(torch.bfloat16)
     resid = torch.randn(R + 3, H, generator=g).to(torch.bfloat16)
@@ -898,6 +900,24 @@ def test_final_norm_and_readout_at_every_width(R, n_ans, H):
         assert ((best - top).abs() <= top.abs() * 2 ** -8 + bound).all()
     assert torch.equal(bits.cpu().bool(), (best_t > best_f).cpu())
     assert torch.equal(margin.cpu(), (best_t.float() - best_f.float()).cpu())
+
+
+@pytest.mark.parametrize("R", [1, 2, 3, 1001])
+def test_readout_bits_do_not_depend_on_the_other_answers(R):
+    """A score is one sum whatever the number of answers spreads over: the best
+    of the first n answers equals the best of them scored alone, bit for bit."""
+    g = _gen(88 + R)
+    normed = torch.randn(R, 2560, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(17, 2560, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    true = (torch.arange(17) % 3 == 0).to(torch.uint8).to(DEV)
+    alone = [K.answer_logits(normed, w[a:a + 1], true[a:a + 1]) for a in range(17)]
+    for n in (1, 2, 3, 4, 5, 8, 9, 17):
+        want = [torch.stack([x[k].float() for x in alone[:n]]).amax(0) for k in (0, 1)]
+        got = K.answer_logits(normed, w[:n], true[:n])
+        bits, margin = K.answer_bits(normed, w[:n], true[:n])
+        assert all(torch.equal(x.float(), y) for x, y in zip(got, want)), n
+        assert torch.equal(bits.bool(), want[0] > want[1])
+        assert torch.equal(margin, want[0] - want[1])
 
 
 # The two tree kernels: "stream" (qh_tree_attention, node pages streamed
