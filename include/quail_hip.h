@@ -278,7 +278,9 @@ int qh_attention_fp8(const void* q, long ldq, int q_rows_total,
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). The call holds no device memory of its own, so calls may
  * overlap on one GPU. At most 131072 sequences per call (QH_E_ARGUMENT
- * beyond). Output bit-identical to qh_attention_fp8.
+ * beyond). Output bit-identical to qh_attention_fp8, which is the faster call
+ * past 256 sequences (1.13 times at 1,500, 1.7 at 4,000): it scans them into its
+ * workspace, where here each wave counts them.
  */
 int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_total,
                              const int64_t* q_rows, const void* k_pool,

@@ -65,6 +65,7 @@ struct AttnParams {
   long ldo;
   float* lse;
   long lse_stride;
+  const int32_t* tile_off;  // [n_seqs + 1] exclusive scan of q-tiles, or nullptr (q_tile)
   // fp8 output (attn_paged_kernel with FP8OUT): e4m3 [n_out, n_q*128] and
   // per-(row, head) scales [n_q, n_out]
   uint8_t* out_q;
@@ -73,6 +74,41 @@ struct AttnParams {
   int n_out;
   int ue8m0;
 };
+
+// Exclusive scan of per-sequence q-tile counts into tile_off[0..n_seqs].
+__global__ __launch_bounds__(1024) void attn_tile_scan_kernel(
+    const int32_t* __restrict__ cu_q, int n_seqs, int32_t* __restrict__ tile_off) {
+  __shared__ int32_t warp_sums[16];
+  __shared__ int32_t carry;
+  if (threadIdx.x == 0) carry = 0;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  for (int base = 0; base < n_seqs; base += 1024) {
+    const int s = base + threadIdx.x;
+    int v = 0;
+    if (s < n_seqs) {
+      const int c = cu_q[s + 1] - cu_q[s];
+      v = c > 0 ? (c + attn::BQ - 1) / attn::BQ : 0;
+    }
+    // inclusive scan within the wave
+    int x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) warp_sums[wid] = x;
+    __syncthreads();
+    int wave_off = 0;
+    for (int w = 0; w < wid; ++w) wave_off += warp_sums[w];
+    const int c0 = carry;
+    if (s < n_seqs) tile_off[s] = c0 + wave_off + x - v;
+    __syncthreads();
+    if (threadIdx.x == 1023) carry = c0 + wave_off + x;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) tile_off[n_seqs] = carry;
+}
 
 // The node-resident tree kernel's two exclusive scans over the segments of
 // cu_a: q-tiles into tile_off[0..n_seg] and work into seg_cost[0..n_seg].
@@ -149,45 +185,114 @@ __global__ __launch_bounds__(1024) void attn_tree_scan_kernel(
   }
 }
 
-// The largest s in [0, n) with key(s) <= b, where key is non-decreasing and
-// key(0) = 0 <= b. A 64-way search: each round the wave's lanes load 64 evenly
-// spaced candidates at once and a ballot picks the last one <= b, so n <= 4096
-// takes two dependent loads where a binary search of scalar loads takes twelve
-// (each an L2 round trip, paid before a workgroup can start its first DMA).
-// Every lane of the wave must call it.
-template <typename T, typename Key>
-__device__ __forceinline__ int last_le_key(int n, T b, int lane, Key key) {
-  int lo = 0, span = n;  // key(lo) <= b; the answer lies in [lo, lo + span)
+// The sequence of q-tile b: the largest s in [0, n) with off[s] <= b, where
+// off is non-decreasing and off[0] = 0 <= b. A 64-way search: each round the
+// wave's lanes load 64 evenly spaced candidates at once and a ballot picks
+// the last one <= b, so n <= 4096 takes two dependent loads where a binary
+// search of scalar loads takes twelve (each an L2 round trip, paid before a
+// workgroup can start its first DMA). Every lane of the wave must call it.
+template <typename T>
+__device__ __forceinline__ int last_le(const T* __restrict__ off, int n, T b, int lane) {
+  int lo = 0, span = n;  // off[lo] <= b; the answer lies in [lo, lo + span)
   while (span > 1) {
     const int step = (span + 63) >> 6;
     const int idx = lo + lane * step;
-    const bool ok = lane * step < span && key(idx) <= b;
+    const bool ok = lane * step < span && off[idx] <= b;
     const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
-    const int k = 63 - __builtin_clzll(m);  // lane 0 always holds (key(lo) <= b)
+    const int k = 63 - __builtin_clzll(m);  // lane 0 always holds (off[lo] <= b)
     lo += k * step;
     span = min(step, span - k * step);
   }
   return __builtin_amdgcn_readfirstlane(lo);
 }
-template <typename T>
-__device__ __forceinline__ int last_le(const T* __restrict__ off, int n, T b, int lane) {
-  return last_le_key<T>(n, b, lane, [&](int i) { return off[i]; });
-}
 __device__ __forceinline__ int tile_seq(const int32_t* __restrict__ off, int n, int b, int lane) {
   return last_le<int32_t>(off, n, b, lane);
 }
 
-// The q-tiles of sequence s occupy slots seq_slot(s) .. of a launch of
-// n_queries / BQ + n_seqs slots: queries ahead of s, in whole tiles, plus one
-// slot per sequence ahead of it, which leaves room for s's own ceil(c / BQ)
-// tiles (floor((a + c) / BQ) - floor(a / BQ) + 1 >= ceil(c / BQ)). The slot is
-// read off cu directly, so no launch ahead of the attention counts tiles (a
-// 4-5 us kernel per layer); the slots between two sequences stay empty.
-__device__ __forceinline__ int seq_slot(const int32_t* __restrict__ cu, int s) {
-  return (int)((uint32_t)(cu[s] - cu[0]) / attn::BQ) + s;
+// A q-tile of a call: BQ queries from query i0 of sequence s, whose `count`
+// queries start at row q0. i0 < 0: the launch holds no such tile.
+struct QTile {
+  int s, q0, count, i0;
+};
+
+// Inclusive sum over the wave's lanes.
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+  return v;
 }
-__device__ __forceinline__ int slot_seq(const int32_t* __restrict__ cu, int n, int b, int lane) {
-  return last_le_key<int>(n, b, lane, [&](int i) { return seq_slot(cu, i); });
+
+// q-tile b of the call, counted over the sequences in order (the heaviest tile
+// of a sequence first): read off `off` where a scan ran ahead, else counted here
+// by each wave for itself. Every lane must call it.
+//
+// Tiles are numbered without gaps: a workgroup that has none comes after all
+// that have one. Workgroups are dealt to XCDs and shader engines in turn, empty
+// or not; numbers read off cu alone (query / 32 + s) leave every second one empty
+// where sequences have 32 queries, and half the engines did the work (us, gaps ->
+// none, 64 heads: 128 sequences of 32 queries over 200-1,024 keys 192 -> 128, of
+// 96 queries 392 -> 325; 1,500 of 32 over 20-200 keys 832 -> 460).
+__device__ __forceinline__ QTile q_tile(const int32_t* __restrict__ cu,
+                                        const int32_t* __restrict__ off, int n, int b, int lane) {
+  using attn::BQ;
+  QTile t{0, 0, 0, -1};
+  if (off != nullptr) {
+    if (b >= off[n]) return t;
+    t.s = tile_seq(off, n, b, lane);
+    t.q0 = cu[t.s];
+    t.count = cu[t.s + 1] - t.q0;
+    t.i0 = ((t.count + BQ - 1) / BQ - 1 - (b - off[t.s])) * BQ;
+    return t;
+  }
+  int left = b;  // tiles ahead of b from sequence s0 on
+  // J blocks of 64 sequences from s0 on; true: b is in one of them
+  auto count = [&](int s0, auto j_c) __attribute__((always_inline)) {
+    constexpr int J = decltype(j_c)::value;
+    int lo[J], hi[J], v[J], sum = 0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int i = s0 + 64 * j + lane;
+      lo[j] = cu[min(i, n)];
+      hi[j] = cu[min(i + 1, n)];
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      v[j] = (max(hi[j] - lo[j], 0) + BQ - 1) / BQ;
+      sum += v[j];
+    }
+    const int all = __builtin_amdgcn_readlane(wave_scan(sum), 63);
+    if (left >= all) {
+      left -= all;
+      return false;
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int end = wave_scan(v[j]);  // tiles up to and with the lane's sequence
+      const int total = __builtin_amdgcn_readlane(end, 63);
+      if (left < total) {
+        // the last lane whose tiles start at or ahead of b: one with tiles
+        const int k = 63 - __builtin_clzll(__builtin_amdgcn_ballot_w64(end - v[j] <= left));
+        t.s = s0 + 64 * j + k;
+        t.q0 = __builtin_amdgcn_readlane(lo[j], k);
+        t.count = __builtin_amdgcn_readlane(hi[j], k) - t.q0;
+        t.i0 = (__builtin_amdgcn_readlane(end, k) - 1 - left) * BQ;
+        break;
+      }
+      left -= total;
+    }
+    return true;
+  };
+  if (n <= 64) {
+    count(0, std::integral_constant<int, 1>{});
+    return t;
+  }
+  for (int s0 = 0; s0 < n; s0 += 512)
+    if (count(s0, std::integral_constant<int, 8>{})) break;
+  return t;
 }
 
 // The work item (q-tile b, head group y) of workgroup (bx, by). The hardware
@@ -245,13 +350,9 @@ __global__ __launch_bounds__(256) void attn_fwd_kernel(AttnParams p) {
   // ---- which sequence and q-tile -------------------------------------------
   int b, hy;
   xcd_item(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, hy);
-  const int s = slot_seq(p.cu_q, p.n_seqs, b, lane);
-  const int q0 = p.cu_q[s];
-  const int count = p.cu_q[s + 1] - q0;
-  const int n_tiles = (count + BQ - 1) / BQ;
-  const int tq = n_tiles - 1 - (b - seq_slot(p.cu_q, s));  // heaviest tile first
-  if (tq < 0) return;
-  const int i0 = tq * BQ;
+  const QTile qt = q_tile(p.cu_q, p.tile_off, p.n_seqs, b, lane);
+  const int s = qt.s, q0 = qt.q0, count = qt.count, i0 = qt.i0;
+  if (i0 < 0) return;
   const int kv_len = p.kv_len[s];
 
   const int group = udiv_uniform(p.n_q, p.n_kv);
@@ -543,11 +644,8 @@ __global__ __launch_bounds__(256, 3) void attn_paged_kernel(AttnParams p) {
   // ---- sequence and q-tile (heaviest tile of a sequence first) -------------
   int b, hy;
   xcd_item(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, hy);
-  const int s = slot_seq(p.cu_q, p.n_seqs, b, lane);
-  const int q0 = p.cu_q[s];
-  const int count = p.cu_q[s + 1] - q0;
-  const int n_qt = (count + BQ - 1) / BQ;
-  const int i0 = (n_qt - 1 - (b - seq_slot(p.cu_q, s))) * BQ;
+  const QTile qt = q_tile(p.cu_q, p.tile_off, p.n_seqs, b, lane);
+  const int s = qt.s, q0 = qt.q0, count = qt.count, i0 = qt.i0;
   if (i0 < 0) return;
   const int kv_len = p.kv_len[s];
   const int group = udiv_uniform(p.n_q, p.n_kv);
@@ -883,9 +981,8 @@ struct TreeParams {
   long ld_out_q;
   float* out_scales;
   int ue8m0;
-  // the node-resident kernel's scans (attn_tree_scan_kernel)
-  const int32_t* tile_off;    // [n_seg + 1] q-tiles
-  const long long* seg_cost;  // [n_seg + 1] work
+  const int32_t* tile_off;    // [n_seg + 1] exclusive scan of q-tiles, or nullptr (q_tile)
+  const long long* seg_cost;  // [n_seg + 1] exclusive scan of work (node-resident kernel)
 };
 
 __device__ __forceinline__ int vswz(int key) { return 4 * (key & 3); }
@@ -906,11 +1003,8 @@ __global__ __launch_bounds__(256, 3) void attn_tree_kernel(TreeParams p) {
   // ---- segment and q-tile (heaviest q-tile of a segment first) -------------
   int b, hy;
   xcd_item(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, b, hy);
-  const int s = slot_seq(p.cu_a, p.n_seg, b, lane);
-  const int q0 = p.cu_a[s];
-  const int count = p.cu_a[s + 1] - q0;
-  const int n_qt = (count + BQ - 1) / BQ;
-  const int i0 = (n_qt - 1 - (b - seq_slot(p.cu_a, s))) * BQ;
+  const QTile qt = q_tile(p.cu_a, p.tile_off, p.n_seg, b, lane);
+  const int s = qt.s, q0 = qt.q0, count = qt.count, i0 = qt.i0;
   if (i0 < 0) return;
   const int group = udiv_uniform(p.n_q, p.n_kv);
   const int hq = hy * HPW + wave;
@@ -926,6 +1020,11 @@ __global__ __launch_bounds__(256, 3) void attn_tree_kernel(TreeParams p) {
   // tile loops they were spilled to VGPR lanes and read back by v_readlane
   int ep_row0 = q0 + i0, ep_rows = count - i0, ep_hq = hq, ep_stage = wave * 32 * 144;
   asm volatile("" : "+v"(ep_row0), "+v"(ep_rows), "+v"(ep_hq), "+v"(ep_stage));
+  // held across the loops (spilled to a VGPR lane if need be): left to the
+  // compiler it was loaded again in every tile, and that load's lgkmcnt(0) waited
+  // for the LDS reads too (8 segments over nodes of 1k-4k keys: 106 us, 110 so)
+  int pool_pages = p.pool_pages;
+  asm volatile("" : "+s"(pool_pages));
 
   // ---- DMA roles: wave (region, pit) moves K (region 0) or V (region 1) of
   // keys 16 pit .. 16 pit + 15 of a tile, as four 1 KiB pieces -------------
@@ -982,7 +1081,7 @@ __global__ __launch_bounds__(256, 3) void attn_tree_kernel(TreeParams p) {
     if (t < n1) {
       const int pidx = 2 * t + pit;
       const bool live = pidx < p.table_width && pidx * PAGE < node_keys && page_id >= 0 &&
-                        page_id < p.pool_pages;
+                        page_id < pool_pages;
       const int slots = live ? min(PAGE, node_keys - pidx * PAGE) : 0;
       const uint32_t bytes = region ? (live ? 4096u : 0u) : (uint32_t)slots * 256u;
       const uint16_t* blk = pool + ((long)(live ? page_id : 0) * p.n_kv + hk) * (PAGE * D);
@@ -1723,11 +1822,10 @@ __global__ __launch_bounds__(512, 1) void attn_tree_node_kernel(TreeParams p) {
 
 using namespace qh;
 
-// The node-resident tree call's scans: tile_off [n_seqs + 1] int32, then
-// seg_cost [n_seqs + 1] int64 at the next 16-byte boundary. The other calls
-// read their q-tiles off cu_q and leave the workspace alone; they ask for
-// paged_workspace_bytes of it all the same, as callers were always told to
-// pass. The query returns what every call needs.
+// tile_off [n_seqs + 1] int32, then (node-resident tree calls) seg_cost
+// [n_seqs + 1] int64 at the next 16-byte boundary. The paged and streaming
+// calls use tile_off only (paged_workspace_bytes), and only past kCountSeqs;
+// the query returns what every call needs.
 static size_t seg_cost_offset(int n_seqs) {
   return ((size_t)(n_seqs + 1) * sizeof(int32_t) + 15) & ~(size_t)15;
 }
@@ -1736,6 +1834,25 @@ static size_t paged_workspace_bytes(int n_seqs) {
 }
 extern "C" size_t qh_attention_workspace_bytes(int n_seqs) {
   return seg_cost_offset(n_seqs) + (size_t)(n_seqs + 1) * sizeof(long long) + 256;
+}
+
+// Up to this many sequences each wave finds its q-tile by itself (q_tile); past
+// it a scan kernel (4-5 us) runs ahead. Time of the call so against with the scan,
+// mean over 1 to 224 queries a sequence, paged / streaming tree: 8 sequences 0.97 /
+// 0.97, 32 0.96 / 0.97, 128 0.98 / 0.98, 200 0.97 / 0.98, 300 0.99 / 0.99, 600 1.02
+// / 1.02, 1,500 1.13 / 1.12, 4,000 1.68 / 1.63.
+constexpr int kCountSeqs = 256;
+alignas(16) static char no_workspace[16];  // a call without one; never dereferenced
+
+// The scan of a paged, contiguous or streaming tree call: its q-tile offsets, or
+// nullptr where the waves count.
+static int tile_scan(const int32_t* cu, int n, void* workspace, hipStream_t st, const char* what,
+                     int32_t** off) {
+  *off = nullptr;
+  if (n <= kCountSeqs || workspace == no_workspace) return QH_OK;
+  *off = (int32_t*)workspace;
+  hipLaunchKernelGGL(attn_tile_scan_kernel, dim3(1), dim3(1024), 0, st, cu, n, *off);
+  return launch_status(what);
 }
 
 // Shared by qh_attention and qh_attention_fp8: checks, tile scan, launch.
@@ -1786,7 +1903,11 @@ static int attention_launch(const void* q, long ldq, int q_rows_total, const int
              "attention: workspace of %zu bytes needed", paged_workspace_bytes(n_seqs));
   QH_REQUIRE(((uintptr_t)workspace & 15) == 0, "attention: workspace must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
+  int32_t* tile_off;
+  const int rc = tile_scan(cu_q, n_seqs, workspace, st, "attention tile scan", &tile_off);
+  if (rc) return rc;
   AttnParams p;
+  p.tile_off = tile_off;
   p.q = (const uint16_t*)q;
   p.ldq = ldq;
   p.q_rows_total = q_rows_total;
@@ -1815,8 +1936,9 @@ static int attention_launch(const void* q, long ldq, int q_rows_total, const int
   p.out_scales = out_scales;
   p.n_out = n_queries;
   p.ue8m0 = ue8m0;
-  const long slots = (long)n_queries / attn::BQ + n_seqs;  // of q-tiles: seq_slot
-  dim3 grid((unsigned)slots, (unsigned)(n_q / attn::HPW));
+  // upper bound on the q-tiles: sum ceil(c/32) <= n_queries/32 + n_seqs
+  const long max_tiles = (long)n_queries / attn::BQ + n_seqs;
+  dim3 grid((unsigned)max_tiles, (unsigned)(n_q / attn::HPW));
   if (paged) {
     if (fp8) {
       if (causal) hipLaunchKernelGGL((attn_paged_kernel<true, true>), grid, dim3(256), 0, st, p);
@@ -1867,12 +1989,9 @@ extern "C" int qh_attention_fp8(const void* q, long ldq, int q_rows_total,
 
 // ---------------------------------------------------------------------------
 // qh_attention_fp8_noalloc: qh_attention_fp8 without a workspace, for callers
-// that cannot allocate. The paged call needs none; the sequence limit is the
-// one this entry point has always had.
-namespace {
+// that cannot allocate: the waves count their q-tiles, however many sequences.
+// The sequence limit is the one this entry point has always had.
 constexpr int kNoAllocSeqs = 131072;  // sequences one call may carry
-alignas(16) char no_workspace[16];    // stands for a workspace; never dereferenced
-}  // namespace
 
 extern "C" int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_total,
                                         const int64_t* q_rows, const void* k_pool,
@@ -1944,16 +2063,17 @@ static int tree_attention_launch(const void* q, long ldq, int n_rows, const void
                "tree_attention_resident: page-table rows of %d pages exceed the %d resident keys",
                table_width, ntree::RES * pattn::BKV);
   }
-  int32_t* tile_off = nullptr;
-  long long* seg_cost = nullptr;
+  int32_t* tile_off = (int32_t*)workspace;
+  long long* seg_cost = (long long*)((char*)workspace + seg_cost_offset(n_seg));
+  int rc;
   if (resident) {
-    tile_off = (int32_t*)workspace;
-    seg_cost = (long long*)((char*)workspace + seg_cost_offset(n_seg));
     hipLaunchKernelGGL(attn_tree_scan_kernel, dim3(1), dim3(1024), 0, st, cu_a, seg_read,
                        read_used, n_reads, n_seg, tile_off, seg_cost);
-    const int rc = launch_status("tree attention tile scan");
-    if (rc) return rc;
+    rc = launch_status("tree attention tile scan");
+  } else {
+    rc = tile_scan(cu_a, n_seg, workspace, st, "tree attention tile scan", &tile_off);
   }
+  if (rc) return rc;
   TreeParams p;
   p.q = (const uint16_t*)q;
   p.ldq = ldq;
@@ -1990,8 +2110,9 @@ static int tree_attention_launch(const void* q, long ldq, int n_rows, const void
     else hipLaunchKernelGGL((attn_tree_node_kernel<false>), grid, dim3(512), 0, st, p);
     return launch_status("tree attention (node resident)");
   }
-  const long slots = (long)n_rows / attn::BQ + n_seg;  // of q-tiles: seq_slot
-  dim3 grid((unsigned)slots, (unsigned)(n_q / attn::HPW));
+  // upper bound on the q-tiles: sum ceil(c/32) <= n_rows/32 + n_seg
+  const long max_tiles = (long)n_rows / attn::BQ + n_seg;
+  dim3 grid((unsigned)max_tiles, (unsigned)(n_q / attn::HPW));
   if (fp8) hipLaunchKernelGGL((attn_tree_kernel<true>), grid, dim3(256), 0, st, p);
   else hipLaunchKernelGGL((attn_tree_kernel<false>), grid, dim3(256), 0, st, p);
   return launch_status("tree attention");

@@ -596,6 +596,62 @@ def test_paged_attention_leaves_rows_of_no_sequence_alone(n_seqs, prefix):
     assert (out[:lo] == 7).all() and (out[hi:] == 7).all()
 
 
+@pytest.mark.parametrize("n_seqs", [1, 2, 63, 64, 65, 200, 256, 257, 511, 513, 1100])
+def test_attention_finds_every_q_tile(n_seqs):
+    """Sequences of 0 to 70 queries, of none at both ends and in runs among
+    them: up to 256 of them the waves count their q-tiles, 64 and 512 at a time,
+    past that a scan runs ahead, without a workspace they always count. Paged,
+    contiguous and streaming tree calls give the bits that calls over 40 of the
+    sequences at a time give, and no workgroup is left without its tile."""
+    g = _gen(700 + n_seqs)
+    n_q, n_kv, scale = 8, 2, 1 / math.sqrt(128)
+    lens = torch.randint(1, 71, (n_seqs,), generator=g)
+    lens[torch.rand(n_seqs, generator=g) < 0.3] = 32
+    if n_seqs > 2:
+        lens[torch.rand(n_seqs, generator=g) < 0.3] = 0
+        lens[[0, n_seqs // 2, n_seqs // 2 + 1, -1]] = 0
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)])
+    T = int(cu[-1])
+    used = lens + torch.randint(0, 40, (n_seqs,), generator=g)
+    node = torch.randint(0, 60, (n_seqs,), generator=g)
+    width = -(-int(max(used.max(), node.max())) // 16)
+    table = torch.randint(0, 50, (n_seqs, width), generator=g).to(torch.int32)
+    rand = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)  # noqa: E731
+    q, k, v = rand(T, n_q, 128), rand(T, n_kv, 128), rand(T, n_kv, 128)
+    kp, vp = rand(50, n_kv, 16, 128), rand(50, n_kv, 128, 16)
+    i32 = lambda x: x.to(torch.int32).to(DEV)  # noqa: E731
+
+    def call(lo, hi):
+        a, b = int(cu[lo]), int(cu[hi])
+        cu_q, tab, keys = i32(cu[lo:hi + 1] - a), table[lo:hi].contiguous().to(DEV), i32(used[lo:hi])
+        args = dict(n_queries=b - a, max_q=int(lens[lo:hi].max()), softmax_scale=scale, causal=True,
+                    n_kv=n_kv)
+        out, _ = K.attention(q[a:b], cu_q, keys, k_pool=kp, v_pool=vp, table=tab, **args)
+        outs = [out, *K.attention_fp8(q[a:b], cu_q, keys, k_pool=kp, v_pool=vp, table=tab, **args)]
+        outs.append(K.attention(q[a:b], cu_q, i32(lens[lo:hi]), k_rows=k[a:b], v_rows=v[a:b],
+                                cu_k=cu_q, **args)[0])
+        read = torch.arange(hi - lo, dtype=torch.int32, device=DEV)
+        outs += K.tree_attention(q[a:b], k[a:b], v[a:b], cu_q, read, softmax_scale=scale, k_pool=kp,
+                                 v_pool=vp, table=tab, used=i32(node[lo:hi]), fp8=True)
+        no_ws = torch.empty_like(outs[1])
+        sc = K.col_major_scales(b - a, n_q * 128, DEV)
+        K._hip.call("qh_attention_fp8_noalloc", q[a:b].data_ptr(), n_q * 128, b - a, None,
+                    kp.data_ptr(), vp.data_ptr(), 50, tab.data_ptr(), width, 16, cu_q.data_ptr(),
+                    keys.data_ptr(), hi - lo, b - a, args["max_q"], n_q, n_kv, 128, scale, 1,
+                    no_ws.data_ptr(), n_q * 128, sc.data_ptr(), 0, K._stream())
+        assert torch.equal(no_ws.view(torch.uint8), outs[1].view(torch.uint8))
+        assert torch.equal(sc, outs[2])
+        return [x.contiguous().view(torch.uint8) for x in outs]
+
+    full = call(0, n_seqs)
+    for lo in range(0, n_seqs, 40):
+        hi = min(n_seqs, lo + 40)
+        a, b = int(cu[lo]), int(cu[hi])
+        if a < b:
+            for i, (x, y) in enumerate(zip(call(lo, hi), full)):
+                assert torch.equal(x, y[a:b]), (i, lo)
+
+
 @pytest.mark.parametrize("causal,gathered", [(True, False), (False, True)])
 @pytest.mark.parametrize("ue8m0", [False, True])
 def test_attention_fp8_matches_quantized_bf16(causal, gathered, ue8m0):
