@@ -55,6 +55,8 @@ const at::Tensor& tensor(PyObject* o, const char* name) {
   if (!THPVariable_Check(o)) throw torch::TypeError(std::string(name) + " must be a tensor");
   return THPVariable_Unpack(o);
 }
+// None gives an undefined tensor, whose pointer is null: also for tensors that
+// an entry point requires, which refuses the null (as a ValueError)
 at::Tensor optional_tensor(PyObject* o, const char* name) {
   return o == Py_None ? at::Tensor() : tensor(o, name);
 }
@@ -174,7 +176,7 @@ PyObject* final_norm(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const int64_t R = idx.numel(), H = hidden.size(1);
   at::Tensor out = rows_like(hidden, R, H, at::kBFloat16);
   QH_CALL(qh_final_norm, ptr(hidden), ptr(residual), (const int64_t*)ptr(idx), R, H,
-          ptr(tensor(v[3], "weight")), (float)real(v[4]), ptr(out), stream());
+          ptr(optional_tensor(v[3], "weight")), (float)real(v[4]), ptr(out), stream());
   return wrap(out);
   END_HANDLE_TH_ERRORS
 }
@@ -190,7 +192,7 @@ PyObject* fused_add_rms_norm(PyObject*, PyObject* const* v, Py_ssize_t n) {
     bad_value("hidden and residual must be contiguous");
   if (hidden.sizes() != residual.sizes()) bad_value("hidden and residual shapes differ");
   QH_CALL(qh_fused_add_rms_norm, ptr(hidden), ptr(residual), hidden.size(0), hidden.size(1),
-          ptr(tensor(v[2], "weight")), (float)real(v[3]), stream());
+          ptr(optional_tensor(v[2], "weight")), (float)real(v[3]), stream());
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
@@ -266,7 +268,7 @@ PyObject* fp8_gemm_qkv_rope(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const Gemm g = gemm_operands(v);
   const at::Tensor& positions = tensor(v[4], "positions");
   const at::Tensor& cos_sin = tensor(v[5], "cos_sin");
-  const at::Tensor &qw = tensor(v[6], "q_weight"), &kw = tensor(v[7], "k_weight");
+  const at::Tensor qw = optional_tensor(v[6], "q_weight"), kw = optional_tensor(v[7], "k_weight");
   const float eps = (float)real(v[8]);
   const int64_t n_q = integer(v[9]), n_kv = integer(v[10]);
   const at::Tensor k_pool = optional_tensor(v[11], "k_pool"), v_pool = optional_tensor(v[12], "v_pool");
@@ -306,9 +308,11 @@ PyObject* attention_fp8(PyObject*, PyObject* const* v, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   arity(n, 13, "attention_fp8");
   const at::Tensor& q3 = tensor(v[0], "q");
-  const at::Tensor &cu_q = tensor(v[1], "cu_q"), &kv_len = tensor(v[2], "kv_len");
+  const at::Tensor& cu_q = tensor(v[1], "cu_q");
+  const at::Tensor kv_len = optional_tensor(v[2], "kv_len");
   const int64_t n_queries = integer(v[3]), max_q = integer(v[4]);
-  const at::Tensor &k_pool = tensor(v[7], "k_pool"), &v_pool = tensor(v[8], "v_pool");
+  const at::Tensor& k_pool = tensor(v[7], "k_pool");
+  const at::Tensor v_pool = optional_tensor(v[8], "v_pool");
   const at::Tensor& table = tensor(v[9], "table");
   const at::Tensor q_rows = optional_tensor(v[11], "q_rows");
   check(q3, at::kBFloat16, "q", 3);
@@ -423,7 +427,7 @@ PyObject* answer_bits(PyObject*, PyObject* const* v, Py_ssize_t n) {
   at::Tensor bits = at::empty({R}, normed.options().dtype(at::kByte)), margin;
   if (truth(v[3])) margin = at::empty({R}, normed.options().dtype(at::kFloat));
   QH_CALL(qh_answer_bits, ptr(normed), R, H, ptr(w), w.size(0),
-          (const uint8_t*)ptr(tensor(v[2], "is_true")), (uint8_t*)ptr(bits), (float*)ptr(margin),
+          (const uint8_t*)ptr(optional_tensor(v[2], "is_true")), (uint8_t*)ptr(bits), (float*)ptr(margin),
           stream());
   return pack({bits, margin});
   END_HANDLE_TH_ERRORS
@@ -437,7 +441,7 @@ PyObject* answer_logits(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const int64_t R = normed.size(0), H = normed.size(1);
   at::Tensor best_t = at::empty({R}, normed.options()), best_f = at::empty({R}, normed.options());
   QH_CALL(qh_answer_logits, ptr(normed), R, H, ptr(w), w.size(0),
-          (const uint8_t*)ptr(tensor(v[2], "is_true")), ptr(best_t), ptr(best_f), stream());
+          (const uint8_t*)ptr(optional_tensor(v[2], "is_true")), ptr(best_t), ptr(best_f), stream());
   return pack({best_t, best_f});
   END_HANDLE_TH_ERRORS
 }

@@ -1226,6 +1226,38 @@ def test_tree_attention_agrees_with_the_two_pass_form():
     assert beyond < 0.05, f"values off by more than one e4m3 step: {beyond}"
 
 
+def test_a_required_tensor_left_out_is_a_value_error():
+    """None for a tensor that an entry point requires is its null pointer: a
+    ValueError from the entry point's own check, and no error where there are
+    no rows to read it for."""
+    z = lambda *s, dt=torch.bfloat16: torch.zeros(*s, dtype=dt, device=DEV)  # noqa: E731
+    one = z(1, dt=torch.int64)
+    a, w = z(1, 128, dt=torch.float8_e4m3fn), z(1536, 128, dt=torch.float8_e4m3fn)
+    sa, sw = K.col_major_scales(1, 128, DEV).zero_(), z(12, 1, dt=torch.float32)
+    norm = z(128)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    pool = z(1, 2, 16, 128), z(1, 2, 128, 16)
+
+    def attention(kv_len=i32(1), v_pool=pool[1], n=1):
+        return K.attention_fp8(z(n, 8, 128), i32(0, n), kv_len, n_queries=n, max_q=n,
+                               softmax_scale=1.0, causal=True, k_pool=pool[0], v_pool=v_pool,
+                               table=z(1, 1, dt=torch.int32), n_kv=2)
+
+    rope = (one, z(8, 128))
+    for call in (lambda: K.final_norm(z(1, 128), z(1, 128), one, None, 1e-6),
+                 lambda: K.fused_add_rms_norm(z(1, 128), z(1, 128), None, 1e-6),
+                 lambda: K.fp8_gemm_qkv_rope(a, sa, w, sw, *rope, None, norm, 1e-6, 8, 2),
+                 lambda: K.fp8_gemm_qkv_rope(a, sa, w, sw, *rope, norm, None, 1e-6, 8, 2),
+                 lambda: attention(kv_len=None), lambda: attention(v_pool=None),
+                 lambda: K.answer_bits(z(1, 128), z(2, 128), None),
+                 lambda: K.answer_logits(z(1, 128), z(2, 128), None)):
+        with pytest.raises(ValueError, match="null pointer|without pools"):
+            call()
+    assert K.final_norm(z(1, 128), z(1, 128), one[:0], None, 1e-6).shape == (0, 128)
+    assert attention(kv_len=None, n=0)[0].shape == (0, 1024)
+    assert K.answer_logits(z(0, 128), z(2, 128), None)[0].shape == (0,)
+
+
 def test_every_entry_point_takes_empty_inputs():
     """Zero rows (an empty chunk, no answer rows, no reads) through every
     entry point: each returns empty outputs of the right shapes and launches
