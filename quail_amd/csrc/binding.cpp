@@ -9,6 +9,7 @@
 // Host code only; the kernels are reached through the C ABI.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_strided.h>
@@ -65,9 +66,21 @@ int64_t integer(PyObject* o) {
   if (v == -1 && PyErr_Occurred()) throw python_error();
   return v;
 }
+// int(o): a count that may come as a float or a 0-d tensor
+int64_t to_int(PyObject* o) {
+  THPObjectPtr n(PyNumber_Long(o));
+  if (!n) throw python_error();
+  return integer(n.get());
+}
+// float(o)
 double real(PyObject* o) {
-  const double v = PyFloat_AsDouble(o);
-  if (v == -1.0 && PyErr_Occurred()) throw python_error();
+  double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) {
+    PyErr_Clear();
+    THPObjectPtr f(PyNumber_Float(o));
+    if (!f) throw python_error();
+    v = PyFloat_AS_DOUBLE(f.get());
+  }
   return v;
 }
 bool truth(PyObject* o) {
@@ -310,7 +323,7 @@ PyObject* attention_fp8(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const at::Tensor& q3 = tensor(v[0], "q");
   const at::Tensor& cu_q = tensor(v[1], "cu_q");
   const at::Tensor kv_len = optional_tensor(v[2], "kv_len");
-  const int64_t n_queries = integer(v[3]), max_q = integer(v[4]);
+  const int64_t n_queries = integer(v[3]), max_q = to_int(v[4]);
   const at::Tensor& k_pool = tensor(v[7], "k_pool");
   const at::Tensor v_pool = optional_tensor(v[8], "v_pool");
   const at::Tensor& table = tensor(v[9], "table");

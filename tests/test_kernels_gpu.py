@@ -1258,6 +1258,30 @@ def test_a_required_tensor_left_out_is_a_value_error():
     assert K.answer_logits(z(0, 128), z(2, 128), None)[0].shape == (0,)
 
 
+def test_counts_and_reals_convert_as_int_and_float_do():
+    """attention_fp8's max_q and scale and the norms' eps go through int() and
+    float(): floats, numpy and 0-d tensor values, and numbers in text."""
+    case = _paged_case(91, 3, 40, 30, n_q=8, n_kv=2)
+    args = dict(n_queries=int(case["cu_q"][-1]), causal=True, n_kv=2,
+                k_pool=layout.k_pool_from_rows(case["k_rows"]).to(DEV),
+                v_pool=layout.v_pool_from_rows(case["v_rows"]).to(DEV), table=case["table"].to(DEV))
+    call = lambda max_q, scale: K.attention_fp8(  # noqa: E731
+        case["q"].to(DEV), case["cu_q"].to(DEV), case["used"].to(DEV), max_q=max_q,
+        softmax_scale=scale, **args)[0].view(torch.uint8)
+    want = call(case["max_q"], 0.125)
+    for max_q, scale in ((float(case["max_q"]), torch.tensor(0.125)),
+                         (torch.tensor(float(case["max_q"])), "0.125")):
+        assert torch.equal(call(max_q, scale), want)
+    x, w = case["q"].to(DEV).view(-1, 1024), torch.ones(1024, dtype=torch.bfloat16, device=DEV)
+    a, b = (K.add_rmsnorm_quant(x, w, eps)[0].view(torch.uint8) for eps in (0.5, "0.5"))
+    assert torch.equal(a, b)
+    for bad in (None, "x"):
+        with pytest.raises((TypeError, ValueError)):
+            call(bad, 0.125)
+        with pytest.raises((TypeError, ValueError)):
+            K.add_rmsnorm_quant(x, w, bad)
+
+
 def test_every_entry_point_takes_empty_inputs():
     """Zero rows (an empty chunk, no answer rows, no reads) through every
     entry point: each returns empty outputs of the right shapes and launches
