@@ -109,12 +109,20 @@ void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 // The current stream of the current device, as torch.cuda.current_stream().
 qh_stream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// An output or workspace, allocated without the GIL as torch.empty does: an
+// allocation may wait for the device.
+at::Tensor empty(at::IntArrayRef sizes, const at::TensorOptions& options) {
+  pybind11::gil_scoped_release no_gil;
+  return at::empty(sizes, options);
+}
 at::Tensor rows_like(const at::Tensor& x, int64_t n, int64_t width, at::ScalarType dtype) {
-  return at::empty({n, width}, x.options().dtype(dtype));
+  return empty({n, width}, x.options().dtype(dtype));
 }
 // fp32 scales stored (width / 128, n), viewed (n, width / 128)
 at::Tensor col_major(const at::Tensor& x, int64_t n, int64_t width) {
-  return at::empty_strided({n, width / kGroup}, {1, n > 1 ? n : 1}, x.options().dtype(at::kFloat));
+  const at::TensorOptions options = x.options().dtype(at::kFloat);
+  pybind11::gil_scoped_release no_gil;
+  return at::empty_strided({n, width / kGroup}, {1, n > 1 ? n : 1}, options);
 }
 
 // Runs one C entry point without the GIL and turns its status into the
@@ -333,7 +341,7 @@ PyObject* attention_fp8(PyObject*, PyObject* const* v, Py_ssize_t n) {
   if (d != kGroup) bad_value("one quant group per head needs head_dim 128");
   at::Tensor q = rows_like(q3, n_queries, n_q * d, kE4m3);
   at::Tensor scales = col_major(q3, n_queries, n_q * d);
-  at::Tensor ws = at::empty({(int64_t)qh_attention_workspace_bytes((int)n_seqs)},
+  at::Tensor ws = empty({(int64_t)qh_attention_workspace_bytes((int)n_seqs)},
                             q3.options().dtype(at::kByte));
   QH_CALL(qh_attention_fp8, ptr(q3), q3.stride(0), q3.size(0), (const int64_t*)ptr(q_rows),
           ptr(k_pool), ptr(v_pool), k_pool.size(0), (const int32_t*)ptr(table), table.size(1),
@@ -369,7 +377,7 @@ PyObject* tree_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const int64_t n_reads = table.defined() ? table.size(0) : 0;
   if (n_reads && (!used.defined() || used.numel() != n_reads))
     bad_value("used must have one entry per page-table row");
-  at::Tensor ws = at::empty({(int64_t)qh_attention_workspace_bytes((int)n_seg)},
+  at::Tensor ws = empty({(int64_t)qh_attention_workspace_bytes((int)n_seg)},
                             q3.options().dtype(at::kByte));
   at::Tensor out, q, scales;
   if (fp8) {
@@ -377,7 +385,7 @@ PyObject* tree_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     q = rows_like(q3, T, n_q * d, kE4m3);
     scales = col_major(q3, T, n_q * d);
   } else {
-    out = at::empty({T, n_q, d}, q3.options());
+    out = empty({T, n_q, d}, q3.options());
   }
   const bool resident = truth(v[12]);
   call(resident ? "qh_tree_attention_resident" : "qh_tree_attention",
@@ -437,8 +445,8 @@ PyObject* answer_bits(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const at::Tensor &normed = tensor(v[0], "normed"), &w = tensor(v[1], "w_ans");
   check(normed, at::kBFloat16, "normed", 2);
   const int64_t R = normed.size(0), H = normed.size(1);
-  at::Tensor bits = at::empty({R}, normed.options().dtype(at::kByte)), margin;
-  if (truth(v[3])) margin = at::empty({R}, normed.options().dtype(at::kFloat));
+  at::Tensor bits = empty({R}, normed.options().dtype(at::kByte)), margin;
+  if (truth(v[3])) margin = empty({R}, normed.options().dtype(at::kFloat));
   QH_CALL(qh_answer_bits, ptr(normed), R, H, ptr(w), w.size(0),
           (const uint8_t*)ptr(optional_tensor(v[2], "is_true")), (uint8_t*)ptr(bits), (float*)ptr(margin),
           stream());
@@ -452,7 +460,7 @@ PyObject* answer_logits(PyObject*, PyObject* const* v, Py_ssize_t n) {
   const at::Tensor &normed = tensor(v[0], "normed"), &w = tensor(v[1], "w_ans");
   check(normed, at::kBFloat16, "normed", 2);
   const int64_t R = normed.size(0), H = normed.size(1);
-  at::Tensor best_t = at::empty({R}, normed.options()), best_f = at::empty({R}, normed.options());
+  at::Tensor best_t = empty({R}, normed.options()), best_f = empty({R}, normed.options());
   QH_CALL(qh_answer_logits, ptr(normed), R, H, ptr(w), w.size(0),
           (const uint8_t*)ptr(optional_tensor(v[2], "is_true")), ptr(best_t), ptr(best_f), stream());
   return pack({best_t, best_f});
