@@ -39,7 +39,7 @@ struct Shape {
   static constexpr int EXTRA = EPI == kQkvRope ? (BR / 128) * 8 * TM * WT * 256
                                : EPI == kSiluQuant ? NR * BM * 4 : 0;
   // weight-block scale rows of the tile, all K blocks
-  static constexpr int NB = EPI == kSiluQuant || (EPI == kQkvRope && BR == 256 && NR == 4) ? 2 : 1;
+  static constexpr int NB = EPI == kSiluQuant || (EPI == kQkvRope && BR == 256) ? 2 : 1;
   static constexpr int SBROW = 4 * MAX_NK;
   static constexpr int SBROWS = BR == 256 ? 2 : 1;
   // The last step reads ahead like the others, into registers that nobody uses:
@@ -54,6 +54,7 @@ struct Shape {
   static_assert(2 * NR * RT % NW == 0 && (NS - 1) * LOADS < 64, "DMA pieces");
   static_assert(EPI == kStoreBf16 || BR == 256 || (EPI == kQkvRope && BR == 128),
                 "a fused epilogue needs whole heads, or the gate and up rows of a group");
+  static_assert(EPI != kQkvRope || NR == 4, "a head's n-tiles lie over four waves, two each");
   static_assert(LDS <= 160 * 1024, "LDS");
   static_assert(NS * STAGE + (SBROWS - 1) * SBROW + SB_END <= LDS, "the read ahead's last scale");
 };
@@ -110,7 +111,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
     if constexpr (EPI == kSiluQuant)
       return u < RT / 2 ? wr * (RT / 2) + u : 8 + wr * (RT / 2) + (u - RT / 2);
     else if constexpr (EPI == kQkvRope)
-      return NR == 8 ? 8 * (wr >> 2) + (wr & 3) + 4 * u : 8 * (u >> 1) + wr + 4 * (u & 1);
+      return 8 * (u >> 1) + wr + 4 * (u & 1);
     else
       return wr * RT + u;
   };
@@ -237,7 +238,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
       pos[j] = (int)p.rope.positions[min(m0 + tok0 + 16 * j + (lane & 15), M - 1)];
     const int head0 = tn * (S::BR / 128);
     const bool is_q = head0 < p.rope.n_q, is_v = head0 >= p.rope.n_q + p.rope.n_kv;
-    const uint16_t* wt = (is_q ? p.rope.q_w : p.rope.k_w) + 16 * (wr & 3) + 4 * g;
+    const uint16_t* wt = (is_q ? p.rope.q_w : p.rope.k_w) + 16 * wr + 4 * g;
     wl = *reinterpret_cast<const uint2*>(wt);
     wh = *reinterpret_cast<const uint2*>(wt + 64);
     if (!is_q && p.rope.row_dst != nullptr) {
@@ -453,14 +454,14 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
         const int ps = pos[j] < 0 ? 0 : (pos[j] >= R.max_pos ? R.max_pos - 1 : pos[j]);
-        const uint16_t* cs = R.cos_sin + (long)ps * 128 + 16 * (wr & 3) + 4 * g;
+        const uint16_t* cs = R.cos_sin + (long)ps * 128 + 16 * wr + 4 * g;
         cr[j] = *reinterpret_cast<const uint2*>(cs);
         sr[j] = *reinterpret_cast<const uint2*>(cs + 64);
       }
       float* sq = reinterpret_cast<float*>(lds + S::BM * S::OROW);
       // u's n-tile as (head of the tile, ib), as ntile() lays them out
-      auto head_of = [&](int u) __attribute__((always_inline)) { return NR == 8 ? wr >> 2 : u >> 1; };
-      const int ib0 = wr & 3;  // u even: n-tile ib0 of its head, u odd: ib0 + 4
+      auto head_of = [](int u) __attribute__((always_inline)) { return u >> 1; };
+      // u even: n-tile wr of its head, u odd: wr + 4
 #pragma unroll
       for (int u = 0; u < RT; ++u)
 #pragma unroll
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(64 * NR * WT, OCC) void fp8_gemm_small_kernel(GemmA
           round_bf16_pair(x0, x1);
           round_bf16_pair(x2, x3);
           v = (f32x4){x0, x1, x2, x3};
-          sq[((head_of(u) * 8 + ib0 + 4 * (u & 1)) * TM * WT + tok0 / 16 + j) * 64 + lane] = sumsq4(x0, x1, x2, x3);
+          sq[((head_of(u) * 8 + wr + 4 * (u & 1)) * TM * WT + tok0 / 16 + j) * 64 + lane] = sumsq4(x0, x1, x2, x3);
         }
       __syncthreads();
 #pragma unroll
