@@ -11,6 +11,19 @@ CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "quail_amd
 CUS = 256
 STORE, SILU, QKV = 0, 1, 2
 
+# epilogue -> its number, weight rows, depth and token counts that take every
+# small tiling for a whole call and for the last tiles of a split one (Qwen3-4B's
+# o, gate_up and qkv projections). The GPU tests run them.
+TILING_CASES = {
+    "store": (STORE, 2560, 4096, (1, 49, 97, 193, 385, 769, 1603, 6403, 6658, 6913, 7363, 8194, 13057,
+                                  19585)),
+    "silu": (SILU, 19456, 2560, (1, 49, 97, 193, 769, 1027, 1537, 1633)),
+    "qkv": (QKV, 6144, 2560, (1, 82, 163, 322, 643, 2689, 2818, 3073, 3394, 5377)),
+}
+# bf16 calls (tokens, weight rows, depth) whose persistent workgroups walk two
+# 256 x 256 tiles and more
+MANY_TILES = [(2333, 19456, 384), (8191, 9728, 1280), (8000, 9728, 1024)]
+
 WRAPPER = """
 #include "gemm_plan.h"
 using namespace qh;
@@ -67,3 +80,28 @@ def test_a_split_launches_every_piece_with_tokens_once_and_no_other(lib, epi, M,
             n = lib.pieces(start, M, N, tokens, rows)
             got = [_pair(lib.piece, start, M, N, tokens, rows, t)[:2] for t in range(n)]
             assert got == want, (tokens, rows, start)
+
+
+def test_the_gpu_tests_sizes_take_every_tiling_whole_and_as_a_tail(lib):
+    """A refit of the cost model that moves a size to another tiling fails here,
+    rather than leave a kernel without a test."""
+    for epilogue, (epi, N, K, sizes) in TILING_CASES.items():
+        taken = set()
+        for M in sizes:
+            large, small, tiles = _pair(lib.plan, epi, M, N, K, CUS)
+            assert large < tiles, (epilogue, M)
+            taken.add((small, large > 0))
+        assert taken == {(i, tail) for i in range(lib.tilings(epi)) for tail in (False, True)}, epilogue
+
+
+def test_the_gpu_tests_many_tiles_are_many(lib):
+    for M, N, K in MANY_TILES:
+        assert _pair(lib.plan, STORE, M, N, K, CUS)[0] >= 2 * CUS, (M, N, K)
+
+
+def test_a_depth_past_the_scale_rows_takes_whole_tiles(lib):
+    for epi, N in ((STORE, 512), (SILU, 512), (QKV, 1536)):
+        for M in (1, 17, 150, 700, 5000):
+            large, _, tiles = _pair(lib.plan, epi, M, N, 256 * 128, CUS)
+            assert large == tiles
+            assert _pair(lib.plan, epi, M, N, 255 * 128, CUS)[0] < tiles or M > 700

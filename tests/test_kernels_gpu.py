@@ -14,6 +14,8 @@ import math
 import pytest
 import torch
 
+from test_gemm_plan import MANY_TILES, TILING_CASES
+
 from oracle import ops as ref
 from quail_amd import kernels as K
 from quail_amd import layout
@@ -195,11 +197,12 @@ def _gemm_inputs(seed, M, N, Kd, dev):
     return a, sa, w, sw
 
 
-@pytest.mark.parametrize("M,N,Kd", [(4096, 4608, 1024), (2333, 19456, 384)])
+@pytest.mark.parametrize("M,N,Kd", [(4096, 4608, 1024), *MANY_TILES])
 def test_fp8_gemm_nt_many_tiles(M, N, Kd):
     """More tiles than compute units: each persistent workgroup walks several
-    tiles, with loads running across tile boundaries. Reference: the same
-    dequantized operands in an fp32 torch matmul on the GPU."""
+    tiles, with loads running across tile boundaries (of the first shape, one
+    tile, with the rest on a smaller tiling). Reference: the same dequantized
+    operands in an fp32 torch matmul on the GPU."""
     a, sa, w, sw = _gemm_inputs(11, M, N, Kd, DEV)
     got = K.fp8_gemm_nt(a, sa, w, sw).float()
     a32 = a.float() * sa.repeat_interleave(128, dim=1)
@@ -374,6 +377,19 @@ def test_fp8_gemm_bits_do_not_depend_on_the_chunk_size(epilogue, Kd, ue8m0):
     for m in TILING_SIZES:
         for i, (x, y) in enumerate(zip(call(m), full)):
             assert torch.equal(x, y[:m]), (m, i)
+
+
+@pytest.mark.parametrize("ue8m0", [False, True])
+@pytest.mark.parametrize("epilogue", ["store", "silu", "qkv"])
+def test_fp8_gemm_every_tiling_whole_and_as_a_tail(epilogue, ue8m0):
+    """Sizes that take every small tiling, for a whole call and for the last
+    tiles of a split one (test_gemm_plan.py checks that they do), against 256 x
+    256 tiles alone, bit for bit."""
+    _, N, Kd, sizes = TILING_CASES[epilogue]
+    call = _gemm_calls(epilogue, max(sizes), Kd, ue8m0, N=None if epilogue == "qkv" else N)
+    for m in sizes:
+        for i, (x, y) in enumerate(zip(call(m), call(m, 256))):
+            assert torch.equal(x, y), (m, i)
 
 
 @pytest.mark.parametrize("ue8m0", [False, True])
