@@ -2004,7 +2004,7 @@ extern "C" int qh_attention_fp8_noalloc(const void* q, long ldq, int q_rows_tota
                                         long ld_out_q, float* scales, int ue8m0,
                                         qh_stream_t stream) {
   QH_REQUIRE(n_seqs >= 0 && n_seqs <= kNoAllocSeqs,
-             "attention_fp8_noalloc: %d sequences; the static scratch holds at most %d",
+             "attention_fp8_noalloc: %d sequences; a call takes at most %d",
              n_seqs, kNoAllocSeqs);
   return qh_attention_fp8(q, ldq, q_rows_total, q_rows, k_pool, v_pool, pool_pages, table,
                           table_width, page_tokens, cu_q, kv_len, n_seqs, n_queries, max_q,

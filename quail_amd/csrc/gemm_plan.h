@@ -140,19 +140,23 @@ struct Pieces {
 // on average and 2 % at most against the best measured one. Against 256 x 256
 // tiles alone (us, Qwen3-4B):
 //   tokens   qkv           o             gate_up       down
-//        1   33.4 ->  8.8  43.0 ->  6.9  31.9 -> 12.4  93.0 -> 11.3
-//       64   34.0 ->  9.3  42.9 ->  8.3  32.7 -> 14.9  94.4 -> 13.9
-//      256   36.6 -> 12.2  44.1 -> 10.7  33.1 -> 21.5  96.0 -> 19.4
-//     1024   37.2 -> 26.3* 44.1 -> 20.4  68.1          96.6 -> 39.6   (* 1000)
-//     2048   40.5          44.2 -> 28.5  103.6         95.8 -> 59.3
+//        1   32.9 ->  8.5  42.6 ->  6.6  32.7 -> 12.3  94.0 -> 11.6
+//       64   33.3 ->  9.0  42.6 ->  7.9  32.4 -> 14.4  94.0 -> 14.2
+//      256   35.4 -> 11.9  43.3 -> 10.6  33.0 -> 22.0  95.8 -> 21.2
+//     1024   37.1 -> 25.8  44.1 -> 20.8  69.6 -> 57.7  96.0 -> 43.0
+//     2048   40.1          44.0 -> 29.7   109 ->  103  96.1 -> 62.2
 // Where the last round of 256 x 256 tiles would leave most of the chip idle,
 // its tiles are cut into small ones in a second launch, which costs 8 us here
 // (its start, and a first round on cold LDS; with 4 two sizes ran up to 4 %
 // slower than unsplit). Tiles and not whole tile rows: gate_up has 76 tiles a
 // row. Measured (us, 256 x 256 tiles alone -> so): gate_up at 1,157 tokens, 380
-// tiles on 256 CUs, 69.3 -> 63.5, at 900 72 -> 58; o at 7,200 tokens, 290 tiles,
-// 99 -> 81; down 225 -> 185, at 14,000 358 -> 328; qkv at 3,000 75 -> 59;
-// Qwen3-32B at 4,000 tokens o 184 -> 154, down 578 -> 482.
+// tiles on 256 CUs, 71.7 -> 66.2, at 900 68 -> 56; o at 7,200 tokens, 290 tiles,
+// 98 -> 75; down 218 -> 160, at 14,000 343 -> 293; qkv at 3,000 76 -> 58;
+// Qwen3-32B at 4,000 tokens o 189 -> 151, down 565 -> 441. A split saves less of
+// a longer call: gate_up's of both models take 0.89 of the unsplit time on
+// average behind one or two whole rounds, 0.93 behind 3 to 5, 0.97 behind 6 to 11,
+// 0.99 behind 12 to 49 and 1.00 past that, where a call's runs differ by 1 to 2 %
+// (to 131,072 tokens; the constants are fitted to 40,000).
 static Plan choose(int epi, int M, int N, int K, int cus) {
   const int all = all_tiles(M, N);
   const int nk = K / gemm::BK;
@@ -180,8 +184,11 @@ static Plan choose(int epi, int M, int N, int K, int cus) {
   // than unsplit at 6,000 tokens and never best)
   const int rounds = all / cus;
   for (int r = rounds; r >= 1 && r >= rounds - (epi == gemm::kSiluQuant ? 0 : 1); --r) {
-    // qkv past two rounds: the split measured -3 to +5 % (its long epilogues
-    // overlap the next tile's start in the persistent kernel)
+    // qkv past two rounds stays whole. The line was drawn when its small tilings'
+    // epilogue was longer and whole tile rows were cut (the split measured -3 to
+    // +5 %). With the present ones it would gain where the last round is short:
+    // -4 to -12 % up to 0.4 of a round, -1.4 to +1.4 % above (130 sizes of 3 to 25
+    // rounds, both models; 11,462 tokens 201 -> 189 us, Qwen3-32B's 6,523 346 -> 304).
     if (epi == gemm::kQkvRope && r > 2) continue;
     if (r * cus < all) with_small(r * cus);
   }

@@ -66,10 +66,10 @@ REJECTED = [
      "multiple of 128"),
     ("qh_group_quant", (None, 128, 4, 100, None, None, 0, None), "multiple of 128"),
     ("qh_e4m3_encode", (None, 6, None, None), "multiple of 4"),
-    # more sequences than the no-allocation entry's static scratch holds
+    # more sequences than the no-allocation entry takes
     ("qh_attention_fp8_noalloc", (None, 4096, 1, None, None, None, 1, None, 1, 16, None, None,
                                   10_000_000, 1, 1, 32, 8, 128, 0.1, 1, None, 4096, None, 0,
-                                  None), "static scratch holds at most"),
+                                  None), "a call takes at most 131072"),
     # a GQA group the tree kernel's head groups cannot tile (6 / 4 heads)
     ("qh_tree_attention", (None, 768, 1, None, None, 512, None, None, 1, None, None, 0, None, 0,
                            None, 0, 16, 6, 4, 128, 0.1, None, 0, None, 0, None, 0, None, 0,

@@ -1,10 +1,10 @@
 """qh_attention_fp8_noalloc against qh_attention_fp8, through the C ABI (MI355X only).
 
-The no-alloc entry point keeps its q-tile scan in a static device array
-instead of a caller workspace. Two calls in a row, the second with fewer
-sequences than the first (the array keeps the first call's scan), must each
-be bit-identical to the workspace entry point on the same inputs, values
-and scales. A call past the array's capacity is refused on the host.
+The no-alloc entry point has no workspace to scan q-tiles into: its waves
+count them. Calls of many and of few sequences, on either side of where the
+workspace entry point scans, must each be bit-identical to it on the same
+inputs, values and scales. A call past the sequence limit is refused on the
+host.
 """
 
 import math
@@ -76,7 +76,8 @@ def _call(c, no_alloc):
 def test_noalloc_attention_matches_the_workspace_entry_point_twice():
     big = _case(71, n_seqs=48, prefix=256, max_suffix=200)
     small = _case(72, n_seqs=5, prefix=40, max_suffix=90)
-    for case in (big, small):
+    scanned = _case(73, n_seqs=300, prefix=40, max_suffix=60)
+    for case in (big, small, scanned):
         want_q, want_s = _call(case, no_alloc=False)
         got_q, got_s = _call(case, no_alloc=True)
         assert torch.equal(got_q, want_q)
@@ -85,7 +86,7 @@ def test_noalloc_attention_matches_the_workspace_entry_point_twice():
 
 
 def test_noalloc_attention_refuses_more_sequences_than_its_scratch_holds():
-    with pytest.raises(ValueError, match="static scratch holds at most 131072"):
+    with pytest.raises(ValueError, match="a call takes at most 131072"):
         _hip.call("qh_attention_fp8_noalloc", None, 4096, 0, None, None, None, 1, None, 1,
                   PAGE, None, None, 131073, 1, 1, N_Q, N_KV, D, 0.1, 1, None, 4096, None, 0,
                   None)
